@@ -38,8 +38,8 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-x", "c++", "-O3", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__",
              "-I/opt/rocm/include", "-ffp-contract=off"]
 
-HIP_SOURCES = ["kernels.hip", "transient_kernels.hip", "noalloc.hip", "dense.hip"]
-CXX_SOURCES = ["symbolic.cpp", "separator.cpp", "api.cpp", "lu.cpp", "circuit.cpp", "transient.cpp"]
+HIP_SOURCES = ["kernels.hip", "transient_kernels.hip", "noalloc.hip", "dense.hip", "fronts.hip"]
+CXX_SOURCES = ["symbolic.cpp", "separator.cpp", "fronts.cpp", "api.cpp", "lu.cpp", "circuit.cpp", "transient.cpp"]
 
 
 def _run(cmd):

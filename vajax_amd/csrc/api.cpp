@@ -137,7 +137,12 @@ int vjx_lu_get_info(const vjx_pattern* pat, vjx_lu_info* o) {
   o->fact_levels = s.n_fact_levels;
   o->fwd_levels = (int32_t)s.fwd.lvl_ptr.size() - 1;
   o->bwd_levels = (int32_t)s.bwd.lvl_ptr.size() - 1;
-  if (!s.fact_band.band_w.empty()) {
+  const int stages = (int)s.front.stage_task.size() - 1;
+  if (s.front.on()) {
+    o->fwd_levels = s.n_fwd_levels;
+    o->bwd_levels = s.n_bwd_levels;
+    o->fact_launches = stages;
+  } else if (!s.fact_band.band_w.empty()) {
     int nlaunch = 0;
     for (size_t b = 0; b + 1 < s.fact_band.band_task.size(); ++b)
       nlaunch += (s.fact_band.band_task[b + 1] > s.fact_band.band_task[b]) +
@@ -148,13 +153,14 @@ int vjx_lu_get_info(const vjx_pattern* pat, vjx_lu_info* o) {
   }
   o->fwd_launches = (int32_t)s.fwd.groups.size();
   o->bwd_launches = (int32_t)s.bwd.groups.size();
+  if (s.front.on()) o->fwd_launches = o->bwd_launches = stages;
   o->n_dense_rows = s.n_dense;
   o->n_offdiag_pivots = s.n_offdiag_pivots;
   o->min_pivot_ratio = s.min_pivot_ratio;
   o->n_blocks = s.n_blocks;
   o->n_block_patterns = s.n_block_patterns;
-  o->fwd_bands = (int32_t)s.fwd_band.band_w.size();
-  o->bwd_bands = (int32_t)s.bwd_band.band_w.size();
+  o->fwd_bands = s.front.on() ? stages : (int32_t)s.fwd_band.band_w.size();
+  o->bwd_bands = s.front.on() ? stages : (int32_t)s.bwd_band.band_w.size();
   o->fwd_hub_rows = (int32_t)s.fwd_band.hub_rows.size();
   o->bwd_hub_rows = (int32_t)s.bwd_band.hub_rows.size();
   for (int k = 0; k < 5; ++k) o->analyze_ms[k] = s.analyze_ms[k];
@@ -459,10 +465,19 @@ int vjx_lu_download(vjx_pattern* pat, double* lu_host) {
     return VJX_ERR_STATE;
   }
   const size_t nnz = pat->lu.sym.col.size();
+  const FrontProgram& F = pat->lu.sym.front;
+  // the front program keeps its factors front by front: LU slots by map
+  std::vector<int32_t> map;
+  if (F.on()) front_slot_map(pat->lu.sym, map);
+  const size_t stored = F.on() ? (size_t)F.storage() : nnz;
   if (pat->lu.factored_prec == VJX_PREC_F32) {
-    std::vector<float> tmp(nnz);
-    VJX_TRY_HIP(hipMemcpy(tmp.data(), pat->lu.lu32.p, nnz * sizeof(float), hipMemcpyDeviceToHost));
-    for (size_t e = 0; e < nnz; ++e) lu_host[e] = tmp[e];
+    std::vector<float> tmp(stored);
+    VJX_TRY_HIP(hipMemcpy(tmp.data(), pat->lu.lu32.p, stored * sizeof(float), hipMemcpyDeviceToHost));
+    for (size_t e = 0; e < nnz; ++e) lu_host[e] = tmp[F.on() ? map[e] : e];
+  } else if (F.on()) {
+    std::vector<double> tmp(stored);
+    VJX_TRY_HIP(hipMemcpy(tmp.data(), pat->lu.lu64.p, stored * sizeof(double), hipMemcpyDeviceToHost));
+    for (size_t e = 0; e < nnz; ++e) lu_host[e] = tmp[map[e]];
   } else {
     VJX_TRY_HIP(hipMemcpy(lu_host, pat->lu.lu64.p, nnz * sizeof(double), hipMemcpyDeviceToHost));
   }

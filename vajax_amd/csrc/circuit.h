@@ -83,6 +83,9 @@ int pattern_autotune_factor(vjx_pattern* pat, const double* data_dev);
 // factors run refine_steps FP64 residual corrections.
 int pattern_solve_async(vjx_pattern* pat, const double* data_dev, const double* rhs, double scale,
                         double* x, int refine_steps);
+// refactorisation (status not reset) and solve together
+int pattern_factor_solve_async(vjx_pattern* pat, const double* data_dev, int prec,
+                               const double* rhs, double scale, double* x, int refine_steps);
 
 void launch_spmv(int n, const int32_t* indptr, const int32_t* indices, const double* data,
                  const double* x, const double* base, double sgn, double* out,

@@ -114,8 +114,21 @@ struct DevBand {
   int lde_bytes = 0;  // dynamic LDS a solve band task may use
 };
 
+// Front program on the device (host plan in sym.front).
+struct DevFronts {
+  DBuf<int32_t> fronts, inst, task, level, idx, asrc, sg_src, sg_div, rs_ptr, rs_rhs,
+      row_single, col_single, us_col, us_chunk;
+  DBuf<uint16_t> apos, cpos, vtab;
+  DBuf<int32_t> kid;
+  DBuf<uint8_t> imap;
+  // update blocks, solve contributions and chunk sums (FP32: as float storage)
+  DBuf<double> cb, cv, part;
+  DBuf<unsigned int> count;  // per column singleton: finished chunks, zero between solves
+};
+
 struct DevLU {
   LuSymbolic sym;
+  DevFronts front;
   bool analyzed = false;
   int factored_prec = -1;  // precision of the current device factors
   DBuf<int32_t> rowptr, col, diag, src, tgt_pos, tgt_seg, upd_l, upd_u, upd_d, l_slot, l_diag, p, q;
@@ -251,6 +264,12 @@ void launch_residual(const ResidualArgs& a, hipStream_t s);
 
 template <typename T>
 void launch_lu_refactor(DevLU& lu, const double* csr, T* lu_vals, DevStatus* st, hipStream_t s);
+// the front program's refactorisation and solve (fronts.hip)
+template <typename T>
+void launch_front_refactor(DevLU& L, const double* csr, T* fac, DevStatus* st, hipStream_t s);
+template <typename T>
+void launch_front_solve(DevLU& L, const T* fac, const double* rhs, double scale, double* x, T* y,
+                        T* z, hipStream_t s);
 // the dense trailing block of a refactorisation (dense.hip)
 template <typename T>
 void launch_dense_block(DevLU& L, T* lu, DevStatus* st, hipStream_t s);
@@ -262,6 +281,12 @@ void launch_dgemm_sub(int M, int N, int Kd, const double* A, int lda, const doub
 template <typename T>
 void launch_lu_solve(DevLU& lu, const T* lu_vals, const double* rhs, double rhs_scale, double* x,
                      T* y, T* z, hipStream_t s, void* const* hub_parts = nullptr);
+// refactorisation and solve of one right-hand side, as a Newton iteration
+// wants them: fewer launches than the two calls where the program allows
+template <typename T>
+void launch_lu_factor_solve(DevLU& lu, const double* csr, T* lu_vals, DevStatus* st,
+                            const double* rhs, double rhs_scale, double* x, T* y, T* z,
+                            hipStream_t s);
 void launch_axpy(int n, double* x, const double* d, hipStream_t s);
 
 void launch_model_eval_raw(int model_id, int count, const double* vb, const double* par,

@@ -2115,6 +2115,10 @@ static void run_fact_groups(DevLU& L, T* lu, DevStatus* st, hipStream_t s) {
 
 template <typename T>
 void launch_lu_refactor(DevLU& L, const double* csr, T* lu, DevStatus* st, hipStream_t s) {
+  if (L.sym.front.on()) {
+    launch_front_refactor<T>(L, csr, lu, st, s);
+    return;
+  }
   const int nnz = (int)L.col.n;
   ktimer_begin(s);
   k_lu_gather<T><<<nblk(nnz, 256), 256, 0, s>>>(nnz, L.src.p, csr, lu, st);
@@ -2192,6 +2196,10 @@ void launch_lu_solve(DevLU& L, const T* lu, const double* rhs, double scale, dou
                      hipStream_t s, void* const* hub_parts) {
   const int n = L.sym.n;
   if (n == 0) return;
+  if (L.sym.front.on()) {
+    launch_front_solve<T>(L, lu, rhs, scale, x, y, z, s);
+    return;
+  }
   k_solve_init<T><<<nblk(n, 256), 256, 0, s>>>(n, L.p.p, rhs, scale, y);
   if (L.fwd_band.on)
     run_tri_bands<T, true>(L, L.sym.fwd_band, L.fwd_band, lu, y, z,

@@ -152,6 +152,43 @@ static hipError_t upload_band(DevBand& d, const BandSchedule& h) {
   return e;
 }
 
+// A vector of plain int32 records.
+template <typename R>
+static hipError_t upload_records(DBuf<int32_t>& d, const std::vector<R>& v) {
+  static_assert(sizeof(R) % sizeof(int32_t) == 0, "records of int32");
+  return d.upload(reinterpret_cast<const int32_t*>(v.data()), v.size() * sizeof(R) / sizeof(int32_t));
+}
+
+static hipError_t upload_fronts(DevFronts& d, const FrontProgram& f) {
+  std::vector<FrontDesc> ordered;  // as the tasks walk them
+  for (int32_t o : f.order) ordered.push_back(f.fronts[o]);
+  hipError_t e = upload_records(d.fronts, ordered);
+  if (e == hipSuccess) e = upload_records(d.inst, f.inst);
+  if (e == hipSuccess) e = d.task.upload(f.task);
+  if (e == hipSuccess) e = d.level.upload(f.level);
+  if (e == hipSuccess) e = d.idx.upload(f.idx);
+  if (e == hipSuccess) e = d.asrc.upload(f.asrc);
+  if (e == hipSuccess) e = upload_records(d.kid, f.kid);
+  if (e == hipSuccess) e = d.imap.upload(f.imap);
+  if (e == hipSuccess) e = d.apos.upload(f.apos);
+  if (e == hipSuccess) e = d.cpos.upload(f.cpos);
+  if (e == hipSuccess) e = d.vtab.upload(f.vtab);
+  if (e == hipSuccess) e = d.sg_src.upload(f.sg_src);
+  if (e == hipSuccess) e = d.sg_div.upload(f.sg_div);
+  if (e == hipSuccess) e = d.rs_ptr.upload(f.rs_ptr);
+  if (e == hipSuccess) e = d.rs_rhs.upload(f.rs_rhs);
+  if (e == hipSuccess) e = d.row_single.upload(f.row_single);
+  if (e == hipSuccess) e = d.col_single.upload(f.col_single);
+  if (e == hipSuccess) e = d.us_col.upload(f.us_col);
+  if (e == hipSuccess) e = d.us_chunk.upload(f.us_chunk);
+  if (e == hipSuccess) e = d.cb.alloc((size_t)f.n_cb);
+  if (e == hipSuccess) e = d.cv.alloc((size_t)f.n_cv);
+  if (e == hipSuccess) e = d.part.alloc(f.us_chunk.size() / 4);
+  if (e == hipSuccess) e = d.count.alloc(f.col_single.size() / 4);
+  if (e == hipSuccess && d.count.n) e = hipMemset(d.count.p, 0, d.count.n * sizeof(unsigned int));
+  return e;
+}
+
 int pattern_upload(vjx_pattern* pat) {
   if (pat->uploaded) return VJX_OK;
   int rc = pattern_upload_csr(pat);
@@ -223,7 +260,9 @@ int pattern_upload(vjx_pattern* pat) {
   VJX_TRY_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
   VJX_TRY_HIP(hipDeviceGetAttribute(&L.n_cu, hipDeviceAttributeMultiprocessorCount, dev));
   L.fwd_band.lde_bytes = L.bwd_band.lde_bytes = std::max(0, lds_max - kTriStaticLds);
-  const size_t nnz = s.col.size();
+  VJX_TRY_HIP(upload_fronts(L.front, s.front));
+  // factor values: the front program's storage, or one per LU slot
+  const size_t nnz = s.front.on() ? (size_t)s.front.storage() : s.col.size();
   const size_t n = (size_t)s.n;
   VJX_TRY_HIP(L.lu64.alloc(nnz));
   VJX_TRY_HIP(L.lu32.alloc(nnz));
@@ -287,10 +326,14 @@ int pattern_autotune_solves(vjx_pattern* pat, const double* data_dev) {
       launch_lu_solve<double>(L, L.lu64.p, L.r64.p, 1.0, L.x64.p, L.y64.p, L.z64.p, s);
   };
   const int candidates[] = {8, 12, 16, 24, 32, 48, 64};
+  // the front program has no band width: one timing of it, at the width the
+  // handle would use
+  const bool front = L.sym.front.on();
   int best = 0;
   float best_ms = 0.f;
   rc = VJX_OK;
   for (int w : candidates) {
+    if (front && w != 16) continue;
     pat->opts.solve_band_width = w;
     lu_rebuild_solve_programs(L.sym, pat->opts);
     hipError_t e = upload_band(L.fwd_band, L.sym.fwd_band);
@@ -385,6 +428,7 @@ int pattern_autotune_factor(vjx_pattern* pat, const double* data_dev) {
       n_widths = 1;
     }
   }
+  if (L.sym.front.on()) n_widths = 1;  // no bands: one timing
   for (int wi = 0; wi < n_widths && rc >= 0; ++wi) {
     const int w = widths[wi];
     if (wi > 0 && w == width0) continue;
@@ -399,7 +443,7 @@ int pattern_autotune_factor(vjx_pattern* pat, const double* data_dev) {
     // faster: plans closer than that trade places from run to run with the
     // timing noise, and another band width also changes the order of the
     // Schur sums (the rounding of the factors)
-    for (int i = 0; i < 3 && rc >= 0; ++i) {
+    for (int i = 0; i < (L.sym.front.on() ? 1 : 3) && rc >= 0; ++i) {
       const int deep = (deep0 + i) % 3;
       L.lu_deep = deep;
       float ms = 0.f;
@@ -444,15 +488,13 @@ int pattern_check_pivots(vjx_pattern* pat) {
   return VJX_OK;
 }
 
-int pattern_solve_async(vjx_pattern* pat, const double* data_dev, const double* rhs, double scale,
+// FP64 refinement of an FP32 solve.
+static int refine_async(vjx_pattern* pat, const double* data_dev, const double* rhs, double scale,
                         double* x, int refine_steps) {
   DevLU& L = pat->lu;
   hipStream_t s = pat->stream;
   const int n = pat->n;
-  if (L.factored_prec == VJX_PREC_F64) {
-    launch_lu_solve<double>(L, L.lu64.p, rhs, scale, x, L.y64.p, L.z64.p, s);
-  } else {
-    launch_lu_solve<float>(L, L.lu32.p, rhs, scale, x, L.y32.p, L.z32.p, s);
+  if (L.factored_prec != VJX_PREC_F64) {
     if (refine_steps > 0) {
       int rc = pattern_upload_csr(pat);
       if (rc < 0) return rc;
@@ -468,6 +510,30 @@ int pattern_solve_async(vjx_pattern* pat, const double* data_dev, const double* 
   }
   VJX_TRY_HIP(hipGetLastError());
   return VJX_OK;
+}
+
+int pattern_solve_async(vjx_pattern* pat, const double* data_dev, const double* rhs, double scale,
+                        double* x, int refine_steps) {
+  DevLU& L = pat->lu;
+  if (L.factored_prec == VJX_PREC_F64)
+    launch_lu_solve<double>(L, L.lu64.p, rhs, scale, x, L.y64.p, L.z64.p, pat->stream);
+  else
+    launch_lu_solve<float>(L, L.lu32.p, rhs, scale, x, L.y32.p, L.z32.p, pat->stream);
+  return refine_async(pat, data_dev, rhs, scale, x, refine_steps);
+}
+
+int pattern_factor_solve_async(vjx_pattern* pat, const double* data_dev, int prec,
+                               const double* rhs, double scale, double* x, int refine_steps) {
+  DevLU& L = pat->lu;
+  if (prec == VJX_PREC_F32)
+    launch_lu_factor_solve<float>(L, data_dev, L.lu32.p, pat->d_status.p, rhs, scale, x, L.y32.p,
+                                  L.z32.p, pat->stream);
+  else
+    launch_lu_factor_solve<double>(L, data_dev, L.lu64.p, pat->d_status.p, rhs, scale, x, L.y64.p,
+                                   L.z64.p, pat->stream);
+  VJX_TRY_HIP(hipGetLastError());
+  L.factored_prec = prec;
+  return refine_async(pat, data_dev, rhs, scale, x, refine_steps);
 }
 
 }  // namespace vjx

@@ -306,18 +306,30 @@ struct Dissector {
 
 }  // namespace
 
+// Vertices with out[v] != 0 are left out of the graph and of the order.
 static void order_columns(int n, const int32_t* indptr, const int32_t* indices, int method,
-                          int leaf, std::vector<int32_t>& order, int& n_dense) {
+                          int leaf, const std::vector<char>& out, std::vector<int32_t>& order,
+                          int& n_dense) {
   Adj adj;
   build_graph(n, indptr, indices, adj);
   std::vector<int32_t> dense = split_dense(n, adj);
   n_dense = (int)dense.size();
+  auto is_out = [&](int v) { return !out.empty() && out[v]; };
+  if (!out.empty()) {
+    dense.erase(std::remove_if(dense.begin(), dense.end(), is_out), dense.end());
+    for (int v = 0; v < n; ++v) {
+      if (out[v])
+        adj[v].clear();
+      else
+        adj[v].erase(std::remove_if(adj[v].begin(), adj[v].end(), is_out), adj[v].end());
+    }
+  }
   std::vector<char> is_dense(n, 0);
   for (int v : dense) is_dense[v] = 1;
   std::vector<int32_t> rest;
   rest.reserve(n);
   for (int v = 0; v < n; ++v)
-    if (!is_dense[v]) rest.push_back(v);
+    if (!is_dense[v] && !is_out(v)) rest.push_back(v);
   order.clear();
   order.reserve(n);
   if (method == 2 || method == 3) {
@@ -348,9 +360,12 @@ struct ColStore {
 
 }  // namespace
 
-// Left-looking LU with threshold partial pivoting (Gilbert-Peierls).
+// Left-looking LU with threshold partial pivoting (Gilbert-Peierls).  pref:
+// per column the row taken as pivot where the threshold allows it (empty: the
+// diagonal).
 static bool gp_factor(int n, const std::vector<int32_t>& cp, const std::vector<int32_t>& ri,
-                      const std::vector<double>& vx, const std::vector<int32_t>& q, double tol,
+                      const std::vector<double>& vx, const std::vector<int32_t>& q,
+                      const std::vector<int32_t>& pref, double tol,
                       int64_t max_nnz, std::vector<int32_t>& pinv, ColStore& L, ColStore& U,
                       int& n_offdiag, double& min_ratio, std::string& err) {
   pinv.assign(n, -1);
@@ -416,7 +431,8 @@ static bool gp_factor(int n, const std::vector<int32_t>& cp, const std::vector<i
       err = "structurally singular matrix at column " + std::to_string(col);
       return false;
     }
-    if (pinv[col] < 0 && mark[col] && std::fabs(x[col]) >= tol * amax) ipiv = col;
+    const int want = pref.empty() ? col : pref[col];
+    if (pinv[want] < 0 && mark[want] && std::fabs(x[want]) >= tol * amax) ipiv = want;
     if (ipiv != col) ++n_offdiag;
     double piv = x[ipiv];
     if (amax > 0.0) min_ratio = std::min(min_ratio, std::fabs(piv) / amax);
@@ -521,6 +537,8 @@ static void rows_by_level(const std::vector<int32_t>& level, SegLen seglen, Leve
   }
 }
 
+// With opt.fronts, a system without a front program returns true with
+// s.plan.ok false and nothing else of use: analyse again without.
 static bool analyze_single(int n, const int32_t* indptr, const int32_t* indices,
                            const double* vals, const AnalyzeOptions& opt, LuSymbolic& s,
                            std::string& err) {
@@ -545,20 +563,77 @@ static bool analyze_single(int n, const int32_t* indptr, const int32_t* indices,
         eid[d] = e;
       }
   }
+  const bool fronts = opt.fronts && opt.band_width > 0 && opt.ordering != 1;
+  Singletons one;
+  std::vector<int32_t> pref;
   if (opt.ordering == 1) {
     s.q.resize(n);
     std::iota(s.q.begin(), s.q.end(), 0);
+  } else if (!fronts) {
+    order_columns(n, indptr, indices, opt.ordering, opt.nd_leaf, {}, s.q, s.n_dense);
   } else {
-    order_columns(n, indptr, indices, opt.ordering, opt.nd_leaf, s.q, s.n_dense);
+    // singletons first, then the fill-reducing order of the rest; a vertex
+    // whose row and column are both gone leaves the graph
+    find_singletons(n, indptr, indices, vals, opt.pivot_tol, one);
+    std::vector<char> row_gone(n, 0), col_gone(n, 0), gone(n, 0);
+    pref.resize(n);
+    std::iota(pref.begin(), pref.end(), 0);
+    for (size_t i = 0; i < one.sc.size(); ++i) {
+      col_gone[one.sc[i]] = row_gone[one.sr[i]] = 1;
+      pref[one.sc[i]] = one.sr[i];
+    }
+    for (size_t i = 0; i < one.rc.size(); ++i) {
+      col_gone[one.rc[i]] = row_gone[one.rr[i]] = 1;
+      pref[one.rc[i]] = one.rr[i];
+    }
+    for (int v = 0; v < n; ++v) gone[v] = row_gone[v] && col_gone[v];
+    std::vector<int32_t> rest;
+    order_columns(n, indptr, indices, opt.ordering, opt.nd_leaf, gone, rest, s.n_dense);
+    s.q = one.sc;
+    s.q.insert(s.q.end(), one.rc.begin(), one.rc.end());
+    for (int v : rest)
+      if (!col_gone[v]) s.q.push_back(v);
   }
   s.analyze_ms[0] = ms_since(t0);
-  s.qinv.assign(n, 0);
-  for (int k = 0; k < n; ++k) s.qinv[s.q[k]] = k;
 
   ColStore L, U;
-  if (!gp_factor(n, cp, ri, vx, s.q, opt.pivot_tol, opt.max_lu_nnz, s.pinv, L, U,
+  if (!gp_factor(n, cp, ri, vx, s.q, pref, opt.pivot_tol, opt.max_lu_nnz, s.pinv, L, U,
                  s.n_offdiag_pivots, s.min_pivot_ratio, err))
     return false;
+  if (fronts) {
+    // the fronts' pivots in consecutive order: renumber the pivots
+    const int ns = (int)(one.sc.size() + one.rc.size());
+    std::vector<int32_t> np;
+    bool ok = true;  // every singleton took its own row
+    for (size_t i = 0; i < one.sr.size() && ok; ++i) ok = s.pinv[one.sr[i]] == (int)i;
+    for (size_t i = 0; i < one.rr.size() && ok; ++i)
+      ok = s.pinv[one.rr[i]] == (int)(one.sr.size() + i);
+    if (!ok || !plan_fronts(n, ns, L.ptr, L.idx, U.ptr, U.idx, s.plan, np)) {
+      s.plan.ok = false;
+      return true;  // the caller analyses again without fronts
+    }
+    s.plan.n_col_single = (int)one.sc.size();
+    s.plan.n_row_single = (int)one.rc.size();
+    std::vector<int32_t> q2(n);
+    for (int k = 0; k < n; ++k) q2[np[k]] = s.q[k];
+    s.q.swap(q2);
+    for (int r = 0; r < n; ++r) s.pinv[r] = np[s.pinv[r]];
+    ColStore L2, U2;
+    std::vector<int32_t> old(n);
+    for (int k = 0; k < n; ++k) old[np[k]] = k;
+    L2.idx.reserve(L.idx.size());
+    U2.idx.reserve(U.idx.size());
+    for (int k = 0; k < n; ++k) {
+      for (int64_t e = L.ptr[old[k]]; e < L.ptr[old[k] + 1]; ++e) L2.idx.push_back(np[L.idx[e]]);
+      for (int64_t e = U.ptr[old[k]]; e < U.ptr[old[k] + 1]; ++e) U2.idx.push_back(np[U.idx[e]]);
+      L2.ptr.push_back((int64_t)L2.idx.size());
+      U2.ptr.push_back((int64_t)U2.idx.size());
+    }
+    std::swap(L, L2);
+    std::swap(U, U2);
+  }
+  s.qinv.assign(n, 0);
+  for (int k = 0; k < n; ++k) s.qinv[s.q[k]] = k;
   s.p.assign(n, 0);
   for (int r = 0; r < n; ++r) s.p[s.pinv[r]] = r;
   s.analyze_ms[1] = ms_since(t0) - s.analyze_ms[0];
@@ -615,6 +690,49 @@ static bool analyze_single(int n, const int32_t* indptr, const int32_t* indices,
     }
 
   s.analyze_ms[2] = ms_since(t0) - s.analyze_ms[0] - s.analyze_ms[1];
+  if (s.plan.ok) {
+    // matrix entries of the fronts, and the statistics of the updates
+    const int ns = s.plan.n_col_single + s.plan.n_row_single;
+    std::vector<int32_t> er, ec, id, nlow(n, 0), level(n, 0), lf(n, 0), lb(n, 0);
+    for (int i = 0; i < n; ++i)
+      for (int e = s.rowptr[i]; e < s.rowptr[i + 1]; ++e) {
+        if (s.col[e] < i) ++nlow[s.col[e]];
+        if (i < ns || s.col[e] < ns || s.src[e] < 0) continue;
+        er.push_back(i);
+        ec.push_back(s.col[e]);
+        id.push_back(s.src[e]);
+      }
+    plan_entries(er, ec, id, s.plan);
+    s.n_updates = 0;
+    s.flops = 0.0;
+    for (int k = 0; k < n; ++k) {
+      const int64_t nl = nlow[k], nu = s.rowptr[k + 1] - s.diag[k] - 1;
+      s.n_updates += nl * nu;
+      s.flops += (double)nl + 2.0 * (double)nl * (double)nu;
+    }
+    // pivot levels (a pivot after every pivot whose L column or U row holds
+    // it) and the row levels of the solves
+    std::vector<int32_t> by_u(n, 0);
+    for (int k = 0; k < n; ++k) {
+      int lv = by_u[k], f = 0;
+      for (int e = s.rowptr[k]; e < s.diag[k]; ++e) {
+        lv = std::max(lv, level[s.col[e]] + 1);
+        f = std::max(f, lf[s.col[e]] + 1);
+      }
+      level[k] = lv;
+      lf[k] = f;
+      for (int e = s.diag[k] + 1; e < s.rowptr[k + 1]; ++e)
+        by_u[s.col[e]] = std::max(by_u[s.col[e]], lv + 1);
+      s.n_fact_levels = std::max(s.n_fact_levels, lv + 1);
+      s.n_fwd_levels = std::max(s.n_fwd_levels, f + 1);
+    }
+    for (int i = n - 1; i >= 0; --i) {
+      for (int e = s.diag[i] + 1; e < s.rowptr[i + 1]; ++e) lb[i] = std::max(lb[i], lb[s.col[e]] + 1);
+      s.n_bwd_levels = std::max(s.n_bwd_levels, lb[i] + 1);
+    }
+    s.analyze_ms[3] = ms_since(t0) - s.analyze_ms[0] - s.analyze_ms[1] - s.analyze_ms[2];
+    return true;
+  }
   // ---- dense trailing block (band programs only) ----
   int s0 = n;  // first dense pivot; n: none
   if (opt.band_width > 0 && opt.dense_min > 0 && n >= 2 * opt.dense_min) {
@@ -1248,6 +1366,7 @@ static bool check_tri_lds(const LuSymbolic& s, const BandSchedule& B, Seg seg, s
 }
 
 bool lu_check_schedules(const LuSymbolic& s, std::string& err) {
+  if (s.front.on()) return check_fronts(s, err);
   const int n = s.n;
   if (!check_tri_lds(s, s.fwd_band,
                      [&](int i) { return std::make_pair((int)s.rowptr[i], (int)s.diag[i]); }, err) ||
@@ -1559,6 +1678,7 @@ static void solve_schedules(LuSymbolic& s, const AnalyzeOptions& opt) {
 }
 
 void lu_rebuild_solve_programs(LuSymbolic& s, const AnalyzeOptions& opt) {
+  if (s.front.on()) return;  // the front program has no band width
   solve_schedules(s, opt);
   make_groups(s.fwd, opt.wide_threshold);
   make_groups(s.bwd, opt.wide_threshold);
@@ -1818,17 +1938,90 @@ static void merge_fact_bands(const std::vector<std::pair<const LuSymbolic*, int3
   }
 }
 
+// The program of a system whose blocks all have front plans: the blocks'
+// plans at their rows (s.rowptr / col / diag / src / p / q laid out), then
+// the singletons of every block.
+static void build_front_program(const std::vector<const LuSymbolic*>& pat,
+                                const std::vector<int32_t>& kind, const std::vector<int32_t>& row0,
+                                const std::vector<std::vector<int32_t>>& entry, LuSymbolic& s) {
+  std::vector<const FrontPlan*> plans;
+  for (const LuSymbolic* b : pat) plans.push_back(&b->plan);
+  FrontProgram& F = s.front;
+  assemble_program(plans, kind, row0, entry, s.n, F);
+  std::vector<char> is_rs(s.n, 0);
+  F.rs_ptr.assign(1, 0);
+  for (size_t c = 0; c < kind.size(); ++c) {
+    const FrontPlan& P = *plans[kind[c]];
+    for (int i = 0; i < P.n_row_single; ++i) is_rs[row0[c] + P.n_col_single + i] = 1;
+    const int nb = pat[kind[c]]->n, ns = P.n_col_single + P.n_row_single;
+    for (int i = 0; i < nb; ++i) {
+      const int r = row0[c] + i;
+      for (int e = s.rowptr[r]; i >= ns && e < s.diag[r]; ++e) {
+        if (!is_rs[s.col[e]]) continue;
+        F.rs_rhs.push_back(s.p[s.col[e]]);
+        F.sg_src.push_back(s.src[e]);
+        F.sg_div.push_back(s.src[s.diag[s.col[e]]]);
+      }
+      F.rs_ptr.push_back((int32_t)F.sg_src.size());
+    }
+  }
+  auto value = [&](int e) {
+    F.sg_src.push_back(s.src[e]);
+    F.sg_div.push_back(-1);
+    return (int32_t)F.sg_src.size() - 1;
+  };
+  for (size_t c = 0; c < kind.size(); ++c) {
+    const FrontPlan& P = *plans[kind[c]];
+    for (int i = 0; i < P.n_row_single; ++i) {
+      const int r = row0[c] + P.n_col_single + i;
+      F.row_single.push_back(r);
+      F.row_single.push_back(value(s.diag[r]));
+    }
+    for (int i = 0; i < P.n_col_single; ++i)
+      for (int32_t v : {row0[c] + i, value(s.diag[row0[c] + i]), 0, 0}) F.col_single.push_back(v);
+  }
+  F.us_first = (int32_t)F.sg_src.size();
+  for (size_t i = 0; i < F.col_single.size() / 4; ++i) {
+    int32_t* cs = &F.col_single[4 * i];
+    cs[2] = (int32_t)F.sg_src.size();
+    for (int e = s.diag[cs[0]] + 1; e < s.rowptr[cs[0] + 1]; ++e) {
+      value(e);
+      F.us_col.push_back(s.q[s.col[e]]);
+    }
+    cs[3] = (int32_t)F.sg_src.size();
+    const int nc = std::max(1, (cs[3] - cs[2] + kHubChunk - 1) / kHubChunk);
+    for (int j = 0; j < nc; ++j)
+      for (int32_t v : {(int32_t)i, cs[2] + j * kHubChunk,
+                        std::min(cs[3], cs[2] + (j + 1) * kHubChunk), nc})
+        F.us_chunk.push_back(v);
+  }
+  tiny_layout(F, s.n);
+}
+
 bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const double* vals,
                 const AnalyzeOptions& opt, LuSymbolic& s, std::string& err) {
   const int nnz = indptr[n];
   if (!csr_validate(n, nnz, indptr, indices, err)) return false;
   std::vector<int32_t> comp;
   const int nc = n > 0 ? pattern_components(n, indptr, indices, comp) : 0;
+  AnalyzeOptions plain = opt;
+  plain.fronts = false;
+  const bool fronts = opt.fronts && opt.band_width > 0 && opt.ordering != 1 && n > 0;
   if (nc <= 1) {
     if (!analyze_single(n, indptr, indices, vals, opt, s, err)) return false;
+    if (fronts && !s.plan.ok) return lu_analyze(n, indptr, indices, vals, plain, s, err);
     s.n_blocks = 1;
     s.n_block_patterns = 1;
     const auto t1 = std::chrono::steady_clock::now();
+    if (s.plan.ok) {
+      std::vector<std::vector<int32_t>> entry(1);
+      entry[0].resize(nnz);
+      std::iota(entry[0].begin(), entry[0].end(), 0);
+      build_front_program({&s}, {0}, {0}, entry, s);
+      s.plan = FrontPlan();
+      s.analyze_ms[4] = ms_since(t1);
+      return true;
+    }
     solve_schedules(s, opt);
     s.analyze_ms[4] = ms_since(t1);
     make_groups(s.fwd, opt.wide_threshold);
@@ -1870,6 +2063,7 @@ bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const doub
     if (!analyze_single((int)b.verts.size(), b.indptr.data(), b.indices.data(), lv.data(), bopt,
                         sym[k], err))
       return false;
+    if (fronts && !sym[k].plan.ok) return lu_analyze(n, indptr, indices, vals, plain, s, err);
   }
   // lay the blocks out one after another
   s = LuSymbolic();
@@ -1912,10 +2106,12 @@ bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const doub
   std::vector<std::pair<const LuSymbolic*, int32_t>> fact_parts;
   std::vector<int32_t> fact_soff;
   int32_t roff = 0, soff = 0, toff = 0, uoff = 0;
-  std::vector<int32_t> gmap;
+  std::vector<int32_t> gmap, row0;
+  std::vector<std::vector<int32_t>> entry;
   for (int c = 0; c < nc; ++c) {
     const LuSymbolic& b = sym[kind[c]];
     const BlockPattern& bp = blk[c];
+    row0.push_back(roff);
     const int nb = b.n;
     // local A entry -> global A entry
     gmap.resize(bp.indices.size());
@@ -1947,6 +2143,7 @@ bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const doub
       s.l_slot.push_back(b.l_slot[e] + soff);
       s.l_diag.push_back(b.l_diag[e] + soff);
     }
+    if (fronts) entry.push_back(gmap);
     bucket_schedule(b.fact, toff, bf);
     fact_parts.push_back({&b, toff});
     fact_soff.push_back(soff);
@@ -1956,6 +2153,8 @@ bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const doub
     s.flops += b.flops;
     s.n_dense += b.n_dense;
     s.n_fact_levels = std::max(s.n_fact_levels, b.n_fact_levels);
+    s.n_fwd_levels = std::max(s.n_fwd_levels, b.n_fwd_levels);
+    s.n_bwd_levels = std::max(s.n_bwd_levels, b.n_bwd_levels);
     s.n_offdiag_pivots += b.n_offdiag_pivots;
     s.min_pivot_ratio = std::min(s.min_pivot_ratio, b.min_pivot_ratio);
     roff += nb;
@@ -1968,6 +2167,17 @@ bool lu_analyze(int n, const int32_t* indptr, const int32_t* indices, const doub
   for (int k = 0; k < n; ++k) {
     s.qinv[s.q[k]] = k;
     s.pinv[s.p[k]] = k;
+  }
+  if (fronts) {
+    const auto t1 = std::chrono::steady_clock::now();
+    std::vector<const LuSymbolic*> pat;
+    for (const auto& b : sym) {
+      pat.push_back(&b);
+      for (int k = 0; k < 4; ++k) s.analyze_ms[k] += b.analyze_ms[k];
+    }
+    build_front_program(pat, kind, row0, entry, s);
+    s.analyze_ms[4] = ms_since(t1);
+    return true;
   }
   merge_schedule(bf, s.fact);
   merge_fact_bands(fact_parts, fact_soff, s);
@@ -2085,6 +2295,14 @@ void dense_lu_host(int K, double* D) {
 template <typename T>
 void lu_refactor_host(const LuSymbolic& s, const double* a, T* lu) {
   const int64_t nnz = s.rowptr[s.n];
+  if (s.front.on()) {
+    std::vector<T> fac((size_t)s.front.storage());
+    std::vector<int32_t> map;
+    fronts_refactor_host<T>(s, a, fac.data());
+    front_slot_map(s, map);
+    for (int64_t e = 0; e < nnz; ++e) lu[e] = fac[map[e]];
+    return;
+  }
   for (int64_t e = 0; e < nnz; ++e) lu[e] = s.src[e] >= 0 ? (T)a[s.src[e]] : (T)0;
   const int nl = (int)s.fact.lvl_ptr.size() - 1;
   auto term = [&](int u) { return lu[s.upd_l[u]] * lu[s.upd_u[u]] / lu[s.upd_d[u]]; };
@@ -2126,6 +2344,15 @@ void lu_refactor_host(const LuSymbolic& s, const double* a, T* lu) {
 template <typename T>
 void lu_solve_host(const LuSymbolic& s, const T* lu, const double* b, double* x) {
   const int n = s.n;
+  if (s.front.on()) {
+    // places outside the LU pattern (padding of the fronts) hold zeros
+    std::vector<T> fac((size_t)s.front.storage(), (T)0);
+    std::vector<int32_t> map;
+    front_slot_map(s, map);
+    for (size_t e = 0; e < map.size(); ++e) fac[map[e]] = lu[e];
+    fronts_solve_host<T>(s, fac.data(), b, x);
+    return;
+  }
   std::vector<T> y(n), z(n);
   for (int i = 0; i < n; ++i) y[i] = (T)b[s.p[i]];
   // Each row's sum depends only on its length class (and, under band

@@ -26,6 +26,8 @@
 #include <string>
 #include <vector>
 
+#include "fronts.h"
+
 namespace vjx {
 
 // One launch of a level program: either a single wide level (grid of blocks)
@@ -186,11 +188,17 @@ struct LuSymbolic {
   int dense_start = -1, dense_k = 0, dense_m = 0;
   std::vector<int32_t> dense_slot, dense_pos, dl_slot, dl_pos, du_slot, du_pos;
   double dense_flops = 0.0;  // 2 K^2 m (contributions) + 2 K^3 / 3 (dense LU)
+  // Front program (fronts.h), used in place of the band programs when the
+  // matrix has one: the update, band, dense and solve programs above are then
+  // empty.  plan: the block pattern's plan, only while the analysis runs.
+  FrontProgram front;
+  FrontPlan plan;
   // statistics
   int64_t nnz_l = 0, nnz_u = 0, n_updates = 0;
   double flops = 0.0;
   int n_dense = 0;
   int n_fact_levels = 0;     // pivot levels of the refactorisation
+  int n_fwd_levels = 0, n_bwd_levels = 0;  // row levels of the solves
   int nd_leaf = 0;           // nested-dissection leaf in use (0: other orderings)
   // analysis time (ms): ordering, pivoting, LU pattern, refactorisation
   // program, solve programs (single-block systems)
@@ -217,6 +225,9 @@ struct AnalyzeOptions {
   int dense_min = 96;
   double dense_density = 0.4;
   int solve_band_width = 0;   // solve bands (0: band_width)
+  // front program where the matrix has one and band_width > 0 (else, and for
+  // the natural order, the band or level programs)
+  bool fronts = true;
   int max_band_tasks = 2048;  // workgroups per band launch
   // abandon the analysis once L + U hold more entries than this (0: no
   // limit); the error text then names the fill limit

@@ -217,10 +217,16 @@ struct Driver {
     launch_noi_apply(c->n_noi_zero, c->noi_zero.p, c->n_noi, c->noi_diag.p, c->noi_rows.p,
                      w.csr.p, w.f.p, s);
     if (prof) VJX_TRY_HIP(hipEventRecord(ev[1], s));
-    int rc = pattern_refactor_async(pat, w.csr.p, cfg->precision, false);
-    if (rc < 0) return rc;
-    if (prof) VJX_TRY_HIP(hipEventRecord(ev[2], s));
-    rc = pattern_solve_async(pat, w.csr.p, w.f.p, -1.0, w.delta.p, cfg->refine_steps);
+    int rc;
+    if (prof) {  // timed apart
+      rc = pattern_refactor_async(pat, w.csr.p, cfg->precision, false);
+      if (rc < 0) return rc;
+      VJX_TRY_HIP(hipEventRecord(ev[2], s));
+      rc = pattern_solve_async(pat, w.csr.p, w.f.p, -1.0, w.delta.p, cfg->refine_steps);
+    } else {
+      rc = pattern_factor_solve_async(pat, w.csr.p, cfg->precision, w.f.p, -1.0, w.delta.p,
+                                      cfg->refine_steps);
+    }
     if (rc < 0) return rc;
     if (prof) {
       VJX_TRY_HIP(hipEventRecord(ev[3], s));
