@@ -189,12 +189,84 @@ struct FrontArgs {
 
 __device__ __forceinline__ bool finite(double v) { return fabs(v) <= 1.7976931348623157e308; }
 
-// Stage 0 of the refactorisation: workgroup = task, one wavefront per front of
-// its levels; the workgroups from n_task on take the singletons' values.
+// Right-hand side of one permuted row in the solve's precision.
 template <typename T>
+__device__ __forceinline__ T rhs_value(const double* __restrict__ rhs, int i, double scale) {
+  const T v = (T)rhs[i];
+  return scale == -1.0 ? -v : v;
+}
+
+// Before a refactorisation that carries a right-hand side along: the
+// singletons' values, and every row's right-hand side less the row singletons'
+// columns, in permuted order, so that a front reads its part in one step.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    k_front_prep(FrontArgs A, int n, int n_rs_entries, const double* __restrict__ csr, T* sg,
+                 const int32_t* __restrict__ p, const double* __restrict__ rhs, double scale, T* y,
+                 DevStatus* st) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  Growth g;
+  unsigned int bad_in = 0;
+  if (i < n) {
+    T v = rhs_value<T>(rhs, p[i], scale);
+    for (int e = A.rs_ptr[i], e1 = A.rs_ptr[i + 1]; e < e1; ++e) {
+      const double a = csr[A.sg_src[e]];
+      if (!finite(a)) ++bad_in;
+      const T l = (T)a / (T)csr[A.sg_div[e]];
+      g.add((double)l);
+      sg[e] = l;
+      v = fmadd(-l, rhs_value<T>(rhs, A.rs_rhs[e], scale), v);
+    }
+    y[i] = v;
+  }
+  // the other singletons' values
+  for (int e = n_rs_entries + i; e < A.n_sg; e += (int)gridDim.x * 256) {
+    const double a = csr[A.sg_src[e]];
+    if (!finite(a)) ++bad_in;
+    sg[e] = (T)a;
+  }
+  if (st) {
+    block_flags(dbits(g.mag), 0, g.bad, &st->maxl_bits, nullptr, &st->nonfinite);
+    __syncthreads();
+    block_flags(0, 0, bad_in, nullptr, nullptr, &st->nonfinite_in);
+  }
+}
+
+// A front's right-hand side, lane = row: prepared values for its pivots, and
+// the children's contributions.
+template <typename T>
+__device__ __forceinline__ T front_rhs(const FrontArgs& A, const FrontDesc& d, const FrontInst& I,
+                                       int lane, int row, const T* y, const T* cv) {
+  T v = lane < d.k ? y[row] : (T)0;
+  const uint16_t* vt = A.vtab + d.vtab + lane;
+  const T* src = cv + I.cv + d.v0;
+  for (int c0 = 0; c0 < d.nv; c0 += 4) {
+    int at[4];
+    T w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      at[u] = (lane < d.m && c0 + u < d.nv) ? vt[(c0 + u) * d.m] : kNoPos;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (at[u] != kNoPos) w[u] = src[at[u]];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (at[u] != kNoPos) v += w[u];
+  }
+  return v;
+}
+
+// Stage 0 of the refactorisation: workgroup = task, one wavefront per front of
+// its levels; the workgroups from n_task on take the singletons' values.  RHS:
+// the forward solve goes along -- a front's columns of L are in LDS when it
+// ends, so its rows of y (k_front_prep's right-hand sides, then the solve's)
+// and its contributions cost a multiply-add per pivot and no memory round of
+// their own (the forward solve by itself, a launch per stage: 93 us at 65k
+// gates).
+template <typename T, bool RHS>
 __global__ void __launch_bounds__(64 * kWaves)
     k_front_small(FrontArgs A, int task0, int n_task, int lds_wave, const double* __restrict__ csr,
-                  T* fac, T* sg, T* cb, DevStatus* st) {
+                  T* fac, T* sg, T* cb, DevStatus* st, T* y, T* cv) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int lane = (int)threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -258,6 +330,10 @@ __global__ void __launch_bounds__(64 * kWaves)
           }
         };
         children(lane);
+        const int row = I.row + d.r0 + lane;
+        T w = (T)0;
+        if constexpr (RHS) w = front_rhs<T>(A, d, I, lane, row, y, cv);
+        T* cvo = cv + I.cv + d.cv;
         double v[NA];
 #pragma unroll
         for (int u = 0; u < NA; ++u)
@@ -308,7 +384,14 @@ __global__ void __launch_bounds__(64 * kWaves)
           for (int j = 0; j < k; ++j) {
             const T x = F[lane + j * ld];
             fo[j * m + lane] = x;
+            if constexpr (RHS) w = fmadd(lane > j ? -x : (T)0, lane_value(w, j), w);
             if (lane > j) g.add((double)x);
+          }
+          if constexpr (RHS) {
+            if (lane < k)
+              y[row] = w;
+            else
+              cvo[lane - k] = w;
           }
           T* dst = lane < k ? fo + k * m + lane : co + lane - k;
           const int step = lane < k ? k : ns;
@@ -337,12 +420,12 @@ constexpr int kKidTable = 64;  // children whose ranges a workgroup keeps in LDS
 // One wavefront per front took 0.45 us per pivot at 56 rows (83 FP64
 // operations and 28 cross-lane reads in one instruction stream, about 1 000
 // cycles); here a thread does at most 33 operations.
-template <typename T>
+template <typename T, bool RHS>
 __global__ void __launch_bounds__(256)
     k_front_large(FrontArgs A, int task0, const double* __restrict__ csr, T* fac, T* cb,
-                  DevStatus* st) {
+                  DevStatus* st, T* y, T* cv) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  __shared__ T colbuf[2][64], rowbuf[2][64];
+  __shared__ T colbuf[2][64], rowbuf[2][65], vbuf[64];
   __shared__ int2 kid_range[kKidTable];
   T* F = reinterpret_cast<T*>(lds_raw);
   const int tid = (int)threadIdx.x;
@@ -379,6 +462,9 @@ __global__ void __launch_bounds__(256)
         pc[u] = A.cpos[d.cpos + tid + 256 * u];
         vc[u] = src[tid + 256 * u];
       }
+    if constexpr (RHS) {
+      if (tid < 64) vbuf[tid] = front_rhs<T>(A, d, I, tid, I.row + d.r0 + tid, y, cv);
+    }
     for (int e = tid, tot = front_lds(d.nt); e < tot; e += 256) F[e] = (T)0;
     if (tid < kKidTable) kid_range[tid] = make_int2(kb, ke);
     T v0 = (T)0;
@@ -417,6 +503,11 @@ __global__ void __launch_bounds__(256)
     }
     T acc[2][8];
     const int i0 = ti - pad, i1 = ti + 32 - pad;  // the thread's rows in the front
+    T w0 = (T)0, w1 = (T)0;                       // their right-hand sides
+    if constexpr (RHS) {
+      if (i0 >= 0) w0 = vbuf[i0];
+      if (i1 >= 0) w1 = vbuf[i1];
+    }
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
       const int j = tj + 8 * b - pad;
@@ -439,6 +530,7 @@ __global__ void __launch_bounds__(256)
         if (ti == (p & 31)) {
 #pragma unroll
           for (int b = pb; b < 8; ++b) rowbuf[par][tj + 8 * b] = acc[pa][b];
+          if (RHS && tj == 0) rowbuf[par][64] = pa == 0 ? w0 : w1;
         }
         lds_barrier();
         const T piv = rowbuf[par][p];
@@ -458,12 +550,30 @@ __global__ void __launch_bounds__(256)
         if (!below0) l0 = (T)0;
         if (!below1) l1 = (T)0;
         if (tj <= pp) u[pb] = (T)0;
+        if constexpr (RHS) {
+          const T wp = rowbuf[par][64];
+          if (pa == 0) w0 = fmadd(-l0, wp, w0);
+          w1 = fmadd(-l1, wp, w1);
+        }
 #pragma unroll
         for (int b = pb; b < 8; ++b) {
           if (pa == 0) acc[0][b] = fmadd(-l0, u[b], acc[0][b]);
           acc[1][b] = fmadd(-l1, u[b], acc[1][b]);
         }
         par ^= 1;
+      }
+    }
+    if constexpr (RHS) {
+      if (tj == 0) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const int i = a ? i1 : i0;
+          if (i < 0 || i >= m) continue;
+          if (i < k)
+            y[I.row + d.r0 + i] = a ? w1 : w0;
+          else
+            cv[I.cv + d.cv + i - k] = a ? w1 : w0;
+        }
       }
     }
     T* fo = fac + I.fac + d.fac;
@@ -494,13 +604,6 @@ __global__ void __launch_bounds__(256)
     __syncthreads();
     block_flags(0, 0, bad_in, nullptr, nullptr, &st->nonfinite_in);
   }
-}
-
-// Right-hand side of one permuted row in the solve's precision.
-template <typename T>
-__device__ __forceinline__ T rhs_value(const double* __restrict__ rhs, int i, double scale) {
-  const T v = (T)rhs[i];
-  return scale == -1.0 ? -v : v;
 }
 
 // Right-hand side of a permuted row less the row singletons' columns.
@@ -590,27 +693,49 @@ __device__ __forceinline__ void task_bwd(const FrontArgs& A, const int4& tk, con
       }
       const T r = reciprocal(piv);
       const T* f2 = f + k * m;
-      for (int j0 = m - 1; j0 >= k; j0 -= 8) {
-        T w[8];
+      // Columns from the last, N at a time; the next N, and at the start the
+      // pivots' own last N, are in flight meanwhile (one round of loads after
+      // another was most of a large front's 7 us).
+      constexpr int N = 8;
+      T c[2][N], e[2][N];
+      auto load_u = [&](T(&w)[N], int j0) {  // update rows' columns j0, j0 - 1, ...
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < N; ++t)
           w[t] = (j0 - t >= k && lane < k) ? f2[(j0 - t - k) * k + lane] : (T)0;
+      };
+      auto load_p = [&](T(&w)[N], int j0) {  // pivots' columns
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < N; ++t) w[t] = lane < j0 - t ? f[(j0 - t) * m + lane] : (T)0;
+      };
+      auto step_u = [&](const T(&w)[N], int j0) {
+#pragma unroll
+        for (int t = 0; t < N; ++t)
           if (j0 - t >= k) v = fmadd(-w[t], lane_value(v, j0 - t), v);
-      }
-      for (int j0 = k - 1; j0 >= 0; j0 -= 8) {
-        T w[8];
+      };
+      auto step_p = [&](const T(&w)[N], int j0) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
-          w[t] = (j0 - t >= 0 && lane < j0 - t) ? f[(j0 - t) * m + lane] : (T)0;
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < N; ++t)
           if (j0 - t >= 0) {
             const T xq = quotient<T>(v, piv, r);
             const T xj = lane_value(xq, j0 - t);
             v = lane == j0 - t ? xq : fmadd(-w[t], xj, v);
           }
+      };
+      load_u(c[0], m - 1);
+      load_p(e[0], k - 1);
+      for (int j0 = m - 1; j0 >= k; j0 -= 2 * N) {
+        if (j0 - N >= k) load_u(c[1], j0 - N);
+        step_u(c[0], j0);
+        if (j0 - N < k) break;
+        if (j0 - 2 * N >= k) load_u(c[0], j0 - 2 * N);
+        step_u(c[1], j0 - N);
+      }
+      for (int j0 = k - 1; j0 >= 0; j0 -= 2 * N) {
+        if (j0 - N >= 0) load_p(e[1], j0 - N);
+        step_p(e[0], j0);
+        if (j0 - N < 0) break;
+        if (j0 - 2 * N >= 0) load_p(e[0], j0 - 2 * N);
+        step_p(e[1], j0 - N);
       }
       if (lane < k) {
         z[row] = v;
@@ -929,55 +1054,53 @@ void launch_tiny(DevLU& L, int mode, const double* csr, T* fac, DevStatus* st, c
 
 }  // namespace
 
+// rhs (may be null): carried along; y then holds the forward solve
 template <typename T>
-void launch_front_refactor(DevLU& L, const double* csr, T* fac, DevStatus* st, hipStream_t s) {
+static void run_refactor(DevLU& L, const double* csr, T* fac, DevStatus* st, const double* rhs,
+                         double scale, T* y, hipStream_t s) {
   const FrontProgram& F = L.sym.front;
   const FrontArgs A = front_args(L);
   T* sg = fac + F.n_fac;
   T* cb = cb_of<T>(L);
-  if (F.tiny.total) {
-    launch_tiny<T>(L, 1, csr, fac, st, nullptr, 1.0, nullptr, s);
-    return;
-  }
+  T* cv = reinterpret_cast<T*>(L.front.cv.p);
   const int ns = (int)F.stage_task.size() - 1;
-  const int nsb = nblk(A.n_sg, 64 * kWaves);
+  const int nsb = rhs ? 0 : nblk(A.n_sg, 64 * kWaves);
+  if (rhs) {
+    ktimer_begin(s);
+    k_front_prep<T><<<nblk(L.sym.n, 256), 256, 0, s>>>(A, L.sym.n, (int)F.rs_rhs.size(), csr, sg,
+                                                       L.p.p, rhs, scale, y, st);
+    ktimer_end(KC_LU_GATHER, s);
+  }
   for (int g = 0; g < std::max(ns, 1); ++g) {
     const int t0 = g < ns ? F.stage_task[g] : 0, nt = g < ns ? F.stage_task[g + 1] - t0 : 0;
     const int grid = nt + (g == 0 ? nsb : 0);
     if (grid == 0) continue;
     const int w = nt > 0 ? front_lds(F.stage_nt[g]) : 0;
+    const size_t lds = sizeof(T) * (size_t)w;
     ktimer_begin(s);
-    if (g == 0)
-      k_front_small<T><<<grid, 64 * kWaves, sizeof(T) * (size_t)w * kWaves, s>>>(
-          A, t0, nt, w, csr, fac, sg, cb, st);
+    if (g == 0 && rhs)
+      k_front_small<T, true><<<grid, 64 * kWaves, lds * kWaves, s>>>(A, t0, nt, w, csr, fac, sg, cb,
+                                                                     st, y, cv);
+    else if (g == 0)
+      k_front_small<T, false><<<grid, 64 * kWaves, lds * kWaves, s>>>(A, t0, nt, w, csr, fac, sg,
+                                                                      cb, st, y, cv);
+    else if (rhs)
+      k_front_large<T, true><<<grid, 256, lds, s>>>(A, t0, csr, fac, cb, st, y, cv);
     else
-      k_front_large<T><<<grid, 256, sizeof(T) * (size_t)w, s>>>(A, t0, csr, fac, cb, st);
+      k_front_large<T, false><<<grid, 256, lds, s>>>(A, t0, csr, fac, cb, st, y, cv);
     ktimer_end(KC_LU_TASKS, s);
   }
 }
 
+// The backward solve and the singletons, from y.
 template <typename T>
-void launch_front_solve(DevLU& L, const T* fac, const double* rhs, double scale, double* x, T* y,
-                        T* z, hipStream_t s) {
+static void run_backward(DevLU& L, const T* fac, double* x, const T* y, T* z, hipStream_t s) {
   const FrontProgram& F = L.sym.front;
   const FrontArgs A = front_args(L);
   const T* sg = fac + F.n_fac;
-  T* cv = reinterpret_cast<T*>(L.front.cv.p);
   T* part = reinterpret_cast<T*>(L.front.part.p);
   const int ns = (int)F.stage_task.size() - 1;
-  if (F.tiny.total) {
-    launch_tiny<T>(L, 2, nullptr, const_cast<T*>(fac), nullptr, rhs, scale, x, s);
-    return;
-  }
-  const int nsb = nblk(A.n_rs + A.n_cs, 64 * kWaves), nrb = nblk(A.n_rs, 64 * kWaves);
-  for (int g = 0; g < std::max(ns, 1); ++g) {
-    const int t0 = g < ns ? F.stage_task[g] : 0, nt = g < ns ? F.stage_task[g + 1] - t0 : 0;
-    const int grid = nt + (g == 0 ? nsb : 0);
-    if (grid == 0) continue;
-    ktimer_begin(s);
-    k_front_fwd<T><<<grid, 64 * kWaves, 0, s>>>(A, t0, nt, fac, sg, L.p.p, rhs, scale, y, cv);
-    ktimer_end(KC_TRI_TASKS, s);
-  }
+  const int nrb = nblk(A.n_rs, 64 * kWaves);
   for (int g = std::max(ns, 1) - 1; g >= 0; --g) {
     const int t0 = g < ns ? F.stage_task[g] : 0, nt = g < ns ? F.stage_task[g + 1] - t0 : 0;
     const int grid = nt + (g == 0 ? nrb : 0);
@@ -997,10 +1120,48 @@ void launch_front_solve(DevLU& L, const T* fac, const double* rhs, double scale,
 }
 
 template <typename T>
+void launch_front_refactor(DevLU& L, const double* csr, T* fac, DevStatus* st, hipStream_t s) {
+  if (L.sym.front.tiny.total) {
+    launch_tiny<T>(L, 1, csr, fac, st, nullptr, 1.0, nullptr, s);
+    return;
+  }
+  run_refactor<T>(L, csr, fac, st, nullptr, 1.0, nullptr, s);
+}
+
+template <typename T>
+void launch_front_solve(DevLU& L, const T* fac, const double* rhs, double scale, double* x, T* y,
+                        T* z, hipStream_t s) {
+  const FrontProgram& F = L.sym.front;
+  if (F.tiny.total) {
+    launch_tiny<T>(L, 2, nullptr, const_cast<T*>(fac), nullptr, rhs, scale, x, s);
+    return;
+  }
+  const FrontArgs A = front_args(L);
+  const T* sg = fac + F.n_fac;
+  T* cv = reinterpret_cast<T*>(L.front.cv.p);
+  const int ns = (int)F.stage_task.size() - 1;
+  const int nsb = nblk(A.n_rs + A.n_cs, 64 * kWaves);
+  for (int g = 0; g < std::max(ns, 1); ++g) {
+    const int t0 = g < ns ? F.stage_task[g] : 0, nt = g < ns ? F.stage_task[g + 1] - t0 : 0;
+    const int grid = nt + (g == 0 ? nsb : 0);
+    if (grid == 0) continue;
+    ktimer_begin(s);
+    k_front_fwd<T><<<grid, 64 * kWaves, 0, s>>>(A, t0, nt, fac, sg, L.p.p, rhs, scale, y, cv);
+    ktimer_end(KC_TRI_TASKS, s);
+  }
+  run_backward<T>(L, fac, x, y, z, s);
+}
+
+template <typename T>
 void launch_lu_factor_solve(DevLU& L, const double* csr, T* fac, DevStatus* st, const double* rhs,
                             double scale, double* x, T* y, T* z, hipStream_t s) {
   if (L.sym.front.on() && L.sym.front.tiny.total) {
     launch_tiny<T>(L, 3, csr, fac, st, rhs, scale, x, s);
+    return;
+  }
+  if (L.sym.front.on()) {
+    run_refactor<T>(L, csr, fac, st, rhs, scale, y, s);
+    run_backward<T>(L, fac, x, y, z, s);
     return;
   }
   launch_lu_refactor<T>(L, csr, fac, st, s);
