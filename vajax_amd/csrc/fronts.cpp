@@ -225,6 +225,7 @@ bool plan_fronts(int n, int n_single, const std::vector<int64_t>& lptr,
   int64_t cb = 0, cv = 0;
   std::vector<int32_t> lpos(n, -1);
   std::vector<uint16_t> pp;
+  std::vector<int32_t> count;  // children's values so far per position
   for (int q = 0; q < nf; ++q) {
     FrontDesc& d = plan.fronts[q];
     const int ld = front_ld(d.nt), s = d.m - d.k;
@@ -237,8 +238,7 @@ bool plan_fronts(int n, int n_single, const std::vector<int64_t>& lptr,
     d.cpos = (int32_t)plan.cpos.size();
     d.v0 = (int32_t)cv;
     d.vtab = (int32_t)plan.vtab.size();
-    d.kid0 = (int32_t)plan.kid.size();
-    d.nkid = (int32_t)kid[q].size();
+    count.assign((size_t)front_lds(d.nt), 0);
     std::vector<std::vector<uint16_t>> contrib(d.m);
     for (int c : kid[q]) {
       FrontDesc& e = plan.fronts[c];
@@ -254,7 +254,7 @@ bool plan_fronts(int n, int n_single, const std::vector<int64_t>& lptr,
       for (size_t a = have - open; a < have && !clash; ++a) {
         const uint16_t x = plan.cpos[d.cpos + a];
         for (size_t b = 0; b < std::min(pp.size(), 64 - open) && !clash; ++b)
-          clash = x != kNoPos && x == pp[b];
+          clash = x != kNoPos && (x & kPosMask) == pp[b];
       }
       if (clash)
         for (size_t a = open; a < 64; ++a) {
@@ -262,11 +262,12 @@ bool plan_fronts(int n, int n_single, const std::vector<int64_t>& lptr,
           ++cb;
         }
       e.cb = (int32_t)cb;
-      plan.kid.push_back({e.cb, sc, (int32_t)plan.imap.size(), 0});
-      plan.imap.resize(plan.imap.size() + d.m, kNoRow);
-      for (int i = 0; i < sc; ++i) plan.imap[plan.kid.back().imap + map[i]] = (uint8_t)i;
       cb += (int64_t)sc * sc;
-      plan.cpos.insert(plan.cpos.end(), pp.begin(), pp.end());
+      for (uint16_t x : pp) {
+        const int nth = count[x]++;
+        d.rounds = std::max(d.rounds, std::min(nth, kMaxRounds) + 1);
+        plan.cpos.push_back((uint16_t)(x | std::min(nth, kMaxRounds - 1) << kPosBits));
+      }
       e.cv = (int32_t)cv;
       for (int i = 0; i < sc; ++i) contrib[map[i]].push_back((uint16_t)(cv - d.v0 + i));
       cv += sc;
@@ -334,14 +335,8 @@ void assemble_program(const std::vector<const FrontPlan*>& plans, const std::vec
       d.a0 += a0[p];
       d.cpos += (int32_t)out.cpos.size();
       d.vtab += (int32_t)out.vtab.size();
-      d.kid0 += (int32_t)out.kid.size();
       out.fronts.push_back(d);
     }
-    for (FrontKid x : P.kid) {
-      x.imap += (int32_t)out.imap.size();
-      out.kid.push_back(x);
-    }
-    out.imap.insert(out.imap.end(), P.imap.begin(), P.imap.end());
     out.idx.insert(out.idx.end(), P.idx.begin(), P.idx.end());
     out.apos.insert(out.apos.end(), P.apos.begin(), P.apos.end());
     out.cpos.insert(out.cpos.end(), P.cpos.begin(), P.cpos.end());
@@ -493,7 +488,7 @@ void assemble_program(const std::vector<const FrontPlan*>& plans, const std::vec
       if (g >= t.stage.size()) continue;
       nt = std::max(nt, t.nt[g]);
       for (const auto& x : t.stage[g])
-        for (int32_t v : {(int32_t)c, x.first, x.second, 0}) out.task.push_back(v);
+        for (int32_t v : {(int32_t)c, x.first, x.second, out.level[x.first]}) out.task.push_back(v);
     }
     out.stage_task.push_back((int32_t)(out.task.size() / 4));
     out.stage_nt.push_back(nt);
@@ -639,8 +634,8 @@ bool check_fronts(const LuSymbolic& s, std::string& err) {
             row_level[r] = l;
           }
           for (int e = 0; e < d.nc; ++e) {
-            const int x = F.cpos[d.cpos + e];
-            if (x != kNoPos && (x % front_ld(d.nt) >= d.m || x / front_ld(d.nt) >= d.m))
+            const int x = F.cpos[d.cpos + e] & kPosMask;
+            if (F.cpos[d.cpos + e] != kNoPos && (x % front_ld(d.nt) >= d.m || x / front_ld(d.nt) >= d.m))
               return fail("update position outside the front");
           }
           for (int e = 0; e < d.na; ++e) {
@@ -652,10 +647,26 @@ bool check_fronts(const LuSymbolic& s, std::string& err) {
           for (int b = 0; b < d.nc; b += 64) {
             std::vector<uint16_t> v(F.cpos.begin() + d.cpos + b,
                                     F.cpos.begin() + d.cpos + std::min(d.nc, b + 64));
+            v.erase(std::remove(v.begin(), v.end(), kNoPos), v.end());
+            for (uint16_t& x : v) x &= kPosMask;
             std::sort(v.begin(), v.end());
-            for (size_t i = 1; i < v.size(); ++i)
-              if (v[i] == v[i - 1] && v[i] != kNoPos) return fail("a group adds to one position twice");
+            if (std::unique(v.begin(), v.end()) != v.end())
+              return fail("a group adds to one position twice");
           }
+          // rounds: every position's values numbered in their order
+          {
+            std::vector<int32_t> seen((size_t)front_lds(d.nt), 0);
+            for (int e = 0; e < d.nc; ++e) {
+              const uint16_t x = F.cpos[d.cpos + e];
+              if (x != kNoPos &&
+                  (x >> kPosBits) != std::min(seen[x & kPosMask]++, kMaxRounds - 1))
+                return fail("a position's values are misnumbered");
+              if (x != kNoPos && (x >> kPosBits) >= d.rounds) return fail("a value past the rounds");
+            }
+            if (*std::max_element(seen.begin(), seen.end()) > kMaxRounds && d.rounds <= kMaxRounds)
+              return fail("more values on a position than rounds");
+          }
+          if (g > 0 && F.level[l + 1] - F.level[l] != 1) return fail("two fronts in a later stage's level");
           if (d.c0 + (int64_t)d.nc > (int64_t)F.n_cb - I.cb ||
               d.v0 < 0 || d.cv + (d.m - d.k) > F.n_cv - I.cv)
             return fail("update block outside the storage");
@@ -705,7 +716,7 @@ void fronts_refactor_host(const LuSymbolic& s, const double* a, T* fac) {
       for (int e = 0; e < d.na; ++e) M[F.apos[d.a0 + e]] = (T)a[F.asrc[d.a0 + I.asrc + e]];
       for (int e = 0; e < d.nc; ++e) {
         const uint16_t p = F.cpos[d.cpos + e];
-        if (p != kNoPos) M[p] += cb[(size_t)I.cb + d.c0 + e];
+        if (p != kNoPos) M[p & kPosMask] += cb[(size_t)I.cb + d.c0 + e];
       }
       for (int p = 0; p < k; ++p) {
         const T piv = M[p + (size_t)p * ld];

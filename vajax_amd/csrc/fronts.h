@@ -44,16 +44,16 @@ struct FrontDesc {
   int32_t v0, nv;   // children's solve contributions from v0 (block), at most nv per row
   int32_t vtab;     // row i's c-th contribution: v0 + FrontProgram::vtab[vtab + c * m + i]
   int32_t nt;       // ceil(m / 8)
-  int32_t kid0, nkid;  // children: FrontProgram::kid
-  int32_t pad0, pad1;
+  int32_t rounds;   // largest number of children's values on one position
+                    // (above kMaxRounds: kMaxRounds + 1)
+  int32_t pad0, pad1, pad2;
 };
 
-// One child of a front: its s x s update block (block) and, per row of the
-// parent, the row's number in the child's block or kNoRow.
-struct FrontKid {
-  int32_t cb, s, imap, pad;
-};
-constexpr uint8_t kNoRow = 0xff;
+// cpos: position, and in the upper bits its number among the children's values
+// on that position, in the children's order.
+constexpr int kPosBits = 13;
+constexpr int kPosMask = (1 << kPosBits) - 1;
+constexpr int kMaxRounds = 7;  // numbers 0 .. 6 (7 marks kNoPos); later ones keep 6
 
 // One diagonal block of the system.
 struct FrontInst {
@@ -69,8 +69,6 @@ struct FrontProgram {
   std::vector<FrontDesc> fronts;
   std::vector<FrontInst> inst;
   std::vector<int32_t> idx;
-  std::vector<FrontKid> kid;
-  std::vector<uint8_t> imap;
   std::vector<uint16_t> apos, cpos, vtab;
   std::vector<int32_t> asrc;  // per instance: matrix entry of each apos
   // Stages, one launch each: a task is a piece of the tree whose children
@@ -80,7 +78,7 @@ struct FrontProgram {
   // with no other child left, by a whole workgroup.
   std::vector<int32_t> stage_task;  // stage g: tasks [stage_task[g], stage_task[g + 1])
   std::vector<int32_t> stage_nt;    // largest nt of the stage
-  std::vector<int32_t> task;        // 4 ints: instance, first level, levels, 0
+  std::vector<int32_t> task;        // 4 ints: instance, first level, levels, first in order
   std::vector<int32_t> level;       // level l: order[level[l] .. level[l + 1])
   std::vector<int32_t> order;       // front ids
   int32_t n_fac = 0, n_cb = 0, n_cv = 0;  // sizes over all instances
@@ -118,8 +116,6 @@ struct FrontPlan {
   std::vector<FrontDesc> fronts;
   std::vector<int32_t> parent;
   std::vector<int32_t> idx;
-  std::vector<FrontKid> kid;
-  std::vector<uint8_t> imap;
   std::vector<uint16_t> apos, cpos, vtab;
   std::vector<int32_t> asrc;  // local matrix entry
   std::vector<int32_t> rows_below;  // pivots in each front's subtree

@@ -108,23 +108,36 @@ struct Growth {
   }
 };
 
-// Elimination of a front's k pivots (at most 32 rows) in the registers of one
-// wavefront, an 8 x 8 grid of lanes; the result goes back to LDS.  A front
-// with fewer than four 8-row tiles uses the last ones (off = 4 - nt), so that
-// every front runs the same code from pivot block off on.
+// Where a front's results go: value (i, j) of its pivots' columns and rows to
+// the factors, the rest to the update block.
 template <typename T>
-__device__ __forceinline__ void front_eliminate(int k, int off, int ld, T* F, int lane) {
+__device__ __forceinline__ T* front_place(int i, int j, int k, int m, T* fo, T* co) {
+  T* const f = fo + (j < k ? j * m + i : k * m + (j - k) * k + i);
+  return (j < k || i < k) ? f : co + (j - k) * (m - k) + (i - k);
+}
+
+// Elimination of a front's k pivots (at most 32 rows) in the registers of one
+// wavefront, an 8 x 8 grid of lanes, from the assembled front in LDS to its
+// places.  A front with fewer than four 8-row tiles uses the last ones (off =
+// 4 - nt), so that every front runs the same code from pivot block off on.  w
+// (RHS): right-hand side, lane = row, before and after.  (Results through LDS
+// and column by column took 200 cycles a column; from the registers a 7-row
+// front is one store.)
+template <bool RHS, typename T>
+__device__ __forceinline__ void front_eliminate(int k, int m, int off, int ld, const T* F, int lane,
+                                                T* fo, T* co, T& w, Growth& g) {
   constexpr int N = kSmallTiles;
   const int ti = lane & 7, tj = lane >> 3;
   // value (ti + 8 (a - off), tj + 8 (b - off)) at base + 8 a + 8 b ld
   const int base = ti - 8 * off + (tj - 8 * off) * ld;
-  T acc[N][N];
+  T acc[N][N], ww[N];
 #pragma unroll
   for (int b = 0; b < N; ++b)
     if (b >= off) {
 #pragma unroll
       for (int a = 0; a < N; ++a)
         if (a >= off) acc[a][b] = F[base + 8 * a + 8 * b * ld];
+      if constexpr (RHS) ww[b] = from_lane(w, 4 * (ti + 8 * (b - off)));
     }
 #pragma unroll
   for (int pb = 0; pb < N; ++pb) {
@@ -144,13 +157,16 @@ __device__ __forceinline__ void front_eliminate(int k, int off, int ld, T* F, in
 #pragma unroll
       for (int a = pb; a < N; ++a) l[a] = quotient<T>(l[a], piv, r);
       const bool below = ti > pp, right = tj > pp, column = tj == pp;
-      if (column) {
 #pragma unroll
-        for (int a = pb; a < N; ++a)
-          if (a > pb || below) acc[a][pb] = l[a];
-      }
+      for (int a = pb; a < N; ++a)
+        if (column && (a > pb || below)) acc[a][pb] = l[a];
       if (!below) l[pb] = (T)0;
       if (!right) u[pb] = (T)0;
+      if constexpr (RHS) {
+        const T wp = lane_value(ww[pb], pp);
+#pragma unroll
+        for (int a = pb; a < N; ++a) ww[a] = fmadd(-l[a], wp, ww[a]);
+      }
 #pragma unroll
       for (int b = pb; b < N; ++b)
 #pragma unroll
@@ -160,10 +176,29 @@ __device__ __forceinline__ void front_eliminate(int k, int off, int ld, T* F, in
 #pragma unroll
   for (int b = 0; b < N; ++b)
     if (b >= off) {
+      const int j = tj + 8 * (b - off);
 #pragma unroll
       for (int a = 0; a < N; ++a)
-        if (a >= off) F[base + 8 * a + 8 * b * ld] = acc[a][b];
+        if (a >= off) {
+          const int i = ti + 8 * (a - off);
+          if (i < m && j < m) {
+            *front_place(i, j, k, m, fo, co) = acc[a][b];
+            if (j < k && i > j) g.add((double)acc[a][b]);
+          }
+        }
     }
+  if constexpr (RHS) {
+    // back to lane = row: row i is held by lane i % 8 (any tj) in ww[i / 8]
+    const int row = lane & 31;
+    T v = (T)0;
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+      if (a >= off) {
+        const T x = from_lane(ww[a], 4 * (row & 7));
+        if ((row >> 3) == a - off) v = x;
+      }
+    w = v;
+  }
 }
 
 struct FrontArgs {
@@ -172,8 +207,6 @@ struct FrontArgs {
   const int4* task;
   const int32_t* level;
   const int32_t* idx;
-  const FrontKid* kid;
-  const uint8_t* imap;
   const uint16_t* apos;
   const uint16_t* cpos;
   const uint16_t* vtab;
@@ -312,7 +345,7 @@ __global__ void __launch_bounds__(64 * kWaves)
           d = A.fronts[o];
           entries(lane);
         }
-        const int k = d.k, m = d.m, ns = m - k, nt = d.nt, ld = front_ld(nt);
+        const int k = d.k, m = d.m, nt = d.nt, ld = front_ld(nt);
         const uint16_t* cpos = A.cpos + d.cpos;
         const T* src = cb + I.cb + d.c0;
         T* fo = fac + I.fac + d.fac;
@@ -359,7 +392,7 @@ __global__ void __launch_bounds__(64 * kWaves)
 #pragma unroll
           for (int u = 0; u < NB; ++u)
             if (pc[u] != kNoPos)
-              __hip_atomic_fetch_add(&F[pc[u]], vc[u], __ATOMIC_RELAXED,
+              __hip_atomic_fetch_add(&F[pc[u] & kPosMask], vc[u], __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_WORKGROUP);
           children(e0 + 64 * NB);
         }
@@ -377,25 +410,12 @@ __global__ void __launch_bounds__(64 * kWaves)
           d = A.fronts[on];
           entries(lane);
         }
-        front_eliminate<T>(k, kSmallTiles - nt, ld, F, lane);
-        wave_sync();
-        // columns out: factors, then the update block, lane = row
-        if (lane < m) {
-          for (int j = 0; j < k; ++j) {
-            const T x = F[lane + j * ld];
-            fo[j * m + lane] = x;
-            if constexpr (RHS) w = fmadd(lane > j ? -x : (T)0, lane_value(w, j), w);
-            if (lane > j) g.add((double)x);
-          }
-          if constexpr (RHS) {
-            if (lane < k)
-              y[row] = w;
-            else
-              cvo[lane - k] = w;
-          }
-          T* dst = lane < k ? fo + k * m + lane : co + lane - k;
-          const int step = lane < k ? k : ns;
-          for (int j = k; j < m; ++j) dst[(j - k) * step] = F[lane + j * ld];
+        front_eliminate<RHS, T>(k, m, kSmallTiles - nt, ld, F, lane, fo, co, w, g);
+        if constexpr (RHS) {
+          if (lane < k)
+            y[row] = w;
+          else if (lane < m)
+            cvo[lane - k] = w;
         }
         wave_sync();
       }
@@ -408,8 +428,6 @@ __global__ void __launch_bounds__(64 * kWaves)
     block_flags(0, 0, bad_in, nullptr, nullptr, &st->nonfinite_in);
   }
 }
-
-constexpr int kKidTable = 64;  // children whose ranges a workgroup keeps in LDS
 
 // A later stage: one front of up to 64 rows per workgroup (or a chain of
 // them).  256 threads hold the front as 32 rows x 8 columns of threads with 2 x
@@ -426,7 +444,6 @@ __global__ void __launch_bounds__(256)
                   DevStatus* st, T* y, T* cv) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ T colbuf[2][64], rowbuf[2][65], vbuf[64];
-  __shared__ int2 kid_range[kKidTable];
   T* F = reinterpret_cast<T*>(lds_raw);
   const int tid = (int)threadIdx.x;
   const int ti = tid & 31, tj = tid >> 5;
@@ -435,26 +452,21 @@ __global__ void __launch_bounds__(256)
   const int4 tk = A.task[task0 + blockIdx.x];
   const FrontInst I = A.inst[tk.x];
   int par = 0;
-  const int oend = A.level[tk.y + tk.z];
-  for (int o = A.level[tk.y]; o < oend; ++o) {
+  const int oend = tk.w + tk.z;  // one front per level
+  for (int o = tk.w; o < oend; ++o) {
     const FrontDesc d = A.fronts[o];
-    const int k = d.k, m = d.m, ns = m - k, ld = front_ld(d.nt), off = 8 - d.nt;
+    const int k = d.k, m = d.m, ld = front_ld(d.nt), off = 8 - d.nt;
     const int pad = 8 * off;  // rows and columns before the front
     // All loads at once: entries' indices and children's values (about 0.6 us
     // away each), then the entries.  Taking the children one after another,
     // map and values, cost 2.2 us per child.
     constexpr int NB = 8;
     const T* src = cb + I.cb + d.c0;
-    int ix = 0, pa0 = 0, pc[NB], kb = 0, ke = 0;
+    int ix = 0, pa0 = 0, pc[NB];
     T vc[NB];
     if (tid < d.na) {
       ix = A.asrc[d.a0 + I.asrc + tid];
       pa0 = A.apos[d.a0 + tid];
-    }
-    if (tid < d.nkid && tid < kKidTable) {
-      const FrontKid kd = A.kid[d.kid0 + tid];
-      kb = kd.cb - d.c0;
-      ke = kb + kd.s * kd.s;
     }
 #pragma unroll
     for (int u = 0; u < NB; ++u)
@@ -466,7 +478,6 @@ __global__ void __launch_bounds__(256)
       if (tid < 64) vbuf[tid] = front_rhs<T>(A, d, I, tid, I.row + d.r0 + tid, y, cv);
     }
     for (int e = tid, tot = front_lds(d.nt); e < tot; e += 256) F[e] = (T)0;
-    if (tid < kKidTable) kid_range[tid] = make_int2(kb, ke);
     T v0 = (T)0;
     if (tid < d.na) {
       const double v = csr[ix];
@@ -481,24 +492,33 @@ __global__ void __launch_bounds__(256)
       F[A.apos[d.a0 + e]] = (T)v;
     }
     lds_barrier();
-    // child by child (fixed sums): a child's values have a place each
-    for (int c = 0; c < d.nkid; ++c) {
-      int2 kr;
-      if (c < kKidTable) {
-        kr = kid_range[c];
-      } else {
-        const FrontKid kd = A.kid[d.kid0 + c];
-        kr = make_int2(kd.cb - d.c0, kd.cb - d.c0 + kd.s * kd.s);
+    // A position's values in the children's order: round c adds the c-th of
+    // each (its number is in the position's upper bits), so a round meets no
+    // position twice and the sums are fixed.  Children one after another, a
+    // barrier each, took 1 000 cycles a child; two or three rounds do.
+    // (A front with more children on one position than there are numbers, a
+    // bus of many blocks, is summed by one wavefront in the program's order.)
+    if (d.rounds > kMaxRounds) {
+      for (int e = tid; tid < 64 && e < d.nc; e += 64) {
+        const int at = A.cpos[d.cpos + e];
+        if (at != kNoPos)
+          __hip_atomic_fetch_add(&F[at & kPosMask], src[e], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
       }
+      lds_barrier();
+    }
+    for (int c = 0; d.rounds <= kMaxRounds && c < d.rounds; ++c) {
 #pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        const int e = tid + 256 * u;
-        if (e >= kr.x && e < kr.y)
-          __hip_atomic_fetch_add(&F[pc[u]], vc[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      for (int u = 0; u < NB; ++u)
+        if (256 * u < d.nc && tid + 256 * u < d.nc && (pc[u] >> kPosBits) == c)
+          __hip_atomic_fetch_add(&F[pc[u] & kPosMask], vc[u], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+      for (int e = 256 * NB + tid; e < d.nc; e += 256) {
+        const int at = A.cpos[d.cpos + e];
+        if ((at >> kPosBits) == c)
+          __hip_atomic_fetch_add(&F[at & kPosMask], src[e], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      for (int e = (kr.x > 256 * NB ? kr.x : 256 * NB) + tid; e < kr.y; e += 256)
-        __hip_atomic_fetch_add(&F[A.cpos[d.cpos + e]], src[e], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
       lds_barrier();
     }
     T acc[2][8];
@@ -580,21 +600,15 @@ __global__ void __launch_bounds__(256)
     T* co = cb + I.cb + d.cb;
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
+      if (b < off) continue;
       const int j = tj + 8 * b - pad;
-      if (j < 0 || j >= m) continue;
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
+        if (a == 0 && off >= 4) continue;  // no rows in the upper half
         const int i = a ? i1 : i0;
-        if (i < 0 || i >= m) continue;
-        const T v = acc[a][b];
-        if (j < k) {
-          fo[j * m + i] = v;
-          if (i > j) g.add((double)v);
-        } else if (i < k) {
-          fo[k * m + (j - k) * k + i] = v;
-        } else {
-          co[(j - k) * ns + i - k] = v;
-        }
+        if (i < 0 || i >= m || j >= m) continue;
+        *front_place(i, j, k, m, fo, co) = acc[a][b];
+        if (j < k && i > j) g.add((double)acc[a][b]);
       }
     }
     if (o + 1 < oend) __syncthreads();  // the chain's next front reads the block
@@ -701,11 +715,12 @@ __device__ __forceinline__ void task_bwd(const FrontArgs& A, const int4& tk, con
       auto load_u = [&](T(&w)[N], int j0) {  // update rows' columns j0, j0 - 1, ...
 #pragma unroll
         for (int t = 0; t < N; ++t)
-          w[t] = (j0 - t >= k && lane < k) ? f2[(j0 - t - k) * k + lane] : (T)0;
+          if (j0 - t >= k) w[t] = lane < k ? f2[(j0 - t - k) * k + lane] : (T)0;
       };
       auto load_p = [&](T(&w)[N], int j0) {  // pivots' columns
 #pragma unroll
-        for (int t = 0; t < N; ++t) w[t] = lane < j0 - t ? f[(j0 - t) * m + lane] : (T)0;
+        for (int t = 0; t < N; ++t)
+          if (j0 - t >= 0) w[t] = lane < j0 - t ? f[(j0 - t) * m + lane] : (T)0;
       };
       auto step_u = [&](const T(&w)[N], int j0) {
 #pragma unroll
@@ -892,6 +907,28 @@ __global__ void __launch_bounds__(64 * kTinyWaves)
   T* y = reinterpret_cast<T*>(lds_raw + S.y);
   if (mode & 2)  // right-hand sides; the row singletons' part follows below
     for (int r = tid; r < S.n_rows; r += nthr) y[r] = rhs_value<T>(rhs, p[r], scale);
+  int32_t* idx = reinterpret_cast<int32_t*>(lds_raw + S.idx);
+  uint16_t* vtab = reinterpret_cast<uint16_t*>(lds_raw + S.vtab);
+  T* cv = reinterpret_cast<T*>(lds_raw + S.cv);
+  T* z = reinterpret_cast<T*>(lds_raw + S.z);
+  FrontArgs B = A;  // the tables in LDS
+  B.fronts = desc;
+  B.level = level - tk.y;
+  B.idx = idx;
+  B.vtab = vtab;
+  if (mode & 2) {
+    for (int i = tid; i < S.n_idx; i += nthr) idx[i] = A.idx[i];
+    for (int i = tid; i < S.n_vtab; i += nthr) vtab[i] = A.vtab[i];
+  }
+  auto core = [&]() {  // the row singletons' part of the right-hand sides
+    for (int r = tid; r < S.n_rows; r += nthr) {
+      T v = y[r];
+      for (int e = A.rs_ptr[r], e1 = A.rs_ptr[r + 1]; e < e1; ++e)
+        v = fmadd(-lsg[e], rhs_value<T>(rhs, A.rs_rhs[e], scale), v);
+      y[r] = v;
+    }
+    __syncthreads();
+  };
   if (mode & 1) {
     double* av = reinterpret_cast<double*>(lds_raw + S.av);
     uint16_t* apos = reinterpret_cast<uint16_t*>(lds_raw + S.apos);
@@ -918,36 +955,34 @@ __global__ void __launch_bounds__(64 * kTinyWaves)
     T* cb = reinterpret_cast<T*>(lds_raw + S.cb);
     T* F = reinterpret_cast<T*>(lds_raw + S.front) + wave * S.lds_wave;
     __syncthreads();
+    if (mode & 2) core();
     for (int lv = 0; lv + 1 < S.n_level; ++lv) {
-      const int f0 = level[0];  // the task's fronts are the program's
       for (int o = level[lv] + wave; o < level[lv + 1]; o += kTinyWaves) {
-        const FrontDesc& d = desc[o - f0];
+        const FrontDesc& d = desc[o];
         const int k = __builtin_amdgcn_readfirstlane(d.k);
         const int m = __builtin_amdgcn_readfirstlane(d.m);
         const int nt = __builtin_amdgcn_readfirstlane(d.nt);
         const int na = d.na, a0 = d.a0, nc = d.nc, cp = d.cpos, c0 = d.c0;
-        const int ns = m - k, ld = front_ld(nt);
+        const int ld = front_ld(nt);
         for (int e = lane, tot = front_lds(nt); e < tot; e += 64) F[e] = (T)0;
         for (int e = lane; e < na; e += 64) F[apos[a0 + e]] = (T)av[a0 + e];
         for (int e = lane; e < nc; e += 64) {
           const int at = cpos[cp + e];
           if (at != kNoPos)
-            __hip_atomic_fetch_add(&F[at], cb[c0 + e], __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(&F[at & kPosMask], cb[c0 + e], __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         wave_sync();
-        front_eliminate<T>(k, kSmallTiles - nt, ld, F, lane);
-        wave_sync();
-        T* fo = lf + d.fac;
-        if (lane < m) {
-          for (int j = 0; j < k; ++j) {
-            const T v = F[lane + j * ld];
-            fo[j * m + lane] = v;
-            if (lane > j) g.add((double)v);
-          }
-          T* dst = lane < k ? fo + k * m + lane : cb + d.cb + lane - k;
-          const int step = lane < k ? k : ns;
-          for (int j = k; j < m; ++j) dst[(j - k) * step] = F[lane + j * ld];
+        // a right-hand side in hand goes along, as in k_front_small
+        T w = (T)0;
+        const int row = I.row + d.r0 + lane;
+        if (mode & 2) w = front_rhs<T>(B, d, I, lane, row, y, cv - I.cv);
+        front_eliminate<true, T>(k, m, kSmallTiles - nt, ld, F, lane, lf + d.fac, cb + d.cb, w, g);
+        if (mode & 2) {
+          if (lane < k)
+            y[row] = w;
+          else if (lane < m)
+            cv[d.cv + lane - k] = w;
         }
         wave_sync();
       }
@@ -959,28 +994,12 @@ __global__ void __launch_bounds__(64 * kTinyWaves)
     for (int i = tid; i < A.n_sg; i += nthr) lsg[i] = sg[i];
   }
   if (mode & 2) {
-    int32_t* idx = reinterpret_cast<int32_t*>(lds_raw + S.idx);
-    uint16_t* vtab = reinterpret_cast<uint16_t*>(lds_raw + S.vtab);
-    T* cv = reinterpret_cast<T*>(lds_raw + S.cv);
-    T* z = reinterpret_cast<T*>(lds_raw + S.z);
-    for (int i = tid; i < S.n_idx; i += nthr) idx[i] = A.idx[i];
-    for (int i = tid; i < S.n_vtab; i += nthr) vtab[i] = A.vtab[i];
-    __syncthreads();
-    for (int r = tid; r < S.n_rows; r += nthr) {
-      T v = y[r];
-      for (int e = A.rs_ptr[r], e1 = A.rs_ptr[r + 1]; e < e1; ++e)
-        v = fmadd(-lsg[e], rhs_value<T>(rhs, A.rs_rhs[e], scale), v);
-      y[r] = v;
+    const T* f0 = lf - I.fac;  // block offsets: one block holds all fronts
+    if (!(mode & 1)) {
+      __syncthreads();
+      core();
+      task_fwd<kTinyWaves, T>(B, tk, f0, [&](int row) { return y[row]; }, y, cv - I.cv);
     }
-    __syncthreads();
-    FrontArgs B = A;
-    B.fronts = desc - level[0];
-    B.level = level - tk.y;
-    B.idx = idx;
-    B.vtab = vtab;
-    // block offsets are the LDS arrays' own (one block holds all fronts)
-    const T* f0 = lf - I.fac;
-    task_fwd<kTinyWaves, T>(B, tk, f0, [&](int row) { return y[row]; }, y, cv - I.cv);
     task_bwd<kTinyWaves, T>(B, tk, f0, q, y, z, x);
     for (int i = tid; i < A.n_rs; i += nthr) {
       const int2 rs = A.row_single[i];
@@ -1012,8 +1031,6 @@ FrontArgs front_args(const DevLU& L) {
   a.task = reinterpret_cast<const int4*>(D.task.p);
   a.level = D.level.p;
   a.idx = D.idx.p;
-  a.kid = reinterpret_cast<const FrontKid*>(D.kid.p);
-  a.imap = D.imap.p;
   a.apos = D.apos.p;
   a.cpos = D.cpos.p;
   a.vtab = D.vtab.p;

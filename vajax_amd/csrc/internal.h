@@ -119,8 +119,6 @@ struct DevFronts {
   DBuf<int32_t> fronts, inst, task, level, idx, asrc, sg_src, sg_div, rs_ptr, rs_rhs,
       row_single, col_single, us_col, us_chunk;
   DBuf<uint16_t> apos, cpos, vtab;
-  DBuf<int32_t> kid;
-  DBuf<uint8_t> imap;
   // update blocks, solve contributions and chunk sums (FP32: as float storage)
   DBuf<double> cb, cv, part;
   DBuf<unsigned int> count;  // per column singleton: finished chunks, zero between solves

@@ -168,8 +168,6 @@ static hipError_t upload_fronts(DevFronts& d, const FrontProgram& f) {
   if (e == hipSuccess) e = d.level.upload(f.level);
   if (e == hipSuccess) e = d.idx.upload(f.idx);
   if (e == hipSuccess) e = d.asrc.upload(f.asrc);
-  if (e == hipSuccess) e = upload_records(d.kid, f.kid);
-  if (e == hipSuccess) e = d.imap.upload(f.imap);
   if (e == hipSuccess) e = d.apos.upload(f.apos);
   if (e == hipSuccess) e = d.cpos.upload(f.cpos);
   if (e == hipSuccess) e = d.vtab.upload(f.vtab);
