@@ -38,9 +38,17 @@ void circuit_build_async(vjx_circuit* c, const double* X, const double* vsrc, co
   for (size_t g = 0; g < c->models.size(); ++g)
     if (only_model < 0 || (size_t)only_model == g) launch_eval(*c->models[g], X, c->d_sc.p, out, s);
   if (only_model < 0) launch_isrc_contrib(c->k, isrc, c->is_dst.p, c->rf.p, c->rq.p, s);
-  if (csr)
-    launch_reduce_jac(c->nse, c->jac_seg.p, c->jac_contrib.p, c->slot_diag.p, c->slot_b.p,
-                      c->d_sc.p, csr, c->hub_slots.view(), s);
+  JacobianArgs j;
+  if (csr) {
+    j.nse = c->nse;
+    j.seg = c->jac_seg.p;
+    j.contrib = c->jac_contrib.p;
+    j.slot_diag = c->slot_diag.p;
+    j.slot_b = c->slot_b.p;
+    j.sc = c->d_sc.p;
+    j.csr = csr;
+    j.hub = c->hub_slots.view();
+  }
   ResidualArgs a;
   a.n_unk = c->n_unk;
   a.m = c->m;
@@ -68,7 +76,7 @@ void circuit_build_async(vjx_circuit* c, const double* X, const double* vsrc, co
   a.I_vs = I_vs;
   a.st = st;
   a.hub = c->hub_rows.view();
-  launch_residual(a, s);
+  launch_stamp(j, a, s);
 }
 
 int circuit_autotune_eval(vjx_circuit* c, const double* X, hipStream_t s) {

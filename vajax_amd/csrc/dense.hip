@@ -24,6 +24,7 @@
 // accumulator rows interleave across the four 16-lane groups.
 #include "block_flags.h"
 #include "internal.h"
+#include "lane_value.h"
 
 namespace vjx {
 
@@ -36,14 +37,6 @@ __device__ __forceinline__ unsigned long long dbits(double x) {
 }
 
 inline int nblk(long long n, int b) { return (int)((n + b - 1) / b); }
-
-// Lane `lane`'s value of v (lane uniform across the wavefront).
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)bits, lane);
-  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(bits >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
 
 // C[M x N] -= A[M x Kd] B[Kd x N]: one 32 x 32 tile of C per workgroup; each
 // of its four wavefronts accumulates the whole tile (2 x 2 blocks of

@@ -12,6 +12,7 @@
 // (a 65k-gate circuit: five).
 #include "block_flags.h"
 #include "internal.h"
+#include "lane_value.h"
 
 #include <algorithm>
 
@@ -24,18 +25,6 @@ constexpr int kSmallTiles = 4;  // 8-row tiles of a front for one wavefront (32 
 
 __device__ __forceinline__ unsigned long long dbits(double x) {
   return (unsigned long long)__double_as_longlong(x);
-}
-
-// Lane `lane`'s value of v (lane uniform across the wavefront).
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)bits, lane);
-  const unsigned int hi =
-      (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(bits >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ float lane_value(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // The value of the lane whose number is addr / 4 (any lane per lane).

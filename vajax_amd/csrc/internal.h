@@ -166,6 +166,8 @@ struct HubChunks {
   double* part3 = nullptr;  // max |.| (residual rows)
   double* part4 = nullptr;  // lim_rhs sums (residual rows of limited circuits)
   double* part5 = nullptr;
+  const int32_t* owner = nullptr;  // chunk c belongs to hub owner[c]
+  unsigned int* count = nullptr;   // per hub: chunks summed so far, zero between launches
   int n_items = 0;
   int n_chunks = 0;
 };
@@ -173,6 +175,8 @@ struct HubChunks {
 struct HubPlan {
   DBuf<int32_t> item, ptr, cs, ce;
   DBuf<double> part, part2, part3, part4, part5;
+  DBuf<int32_t> owner;
+  DBuf<unsigned int> count;
   int n_items = 0, n_chunks = 0;
   // seg: host segment pointers of n segments; nparts: 1, 3 or 5 partial arrays.
   hipError_t build(const int32_t* seg, int n, int nparts);
@@ -187,6 +191,8 @@ struct HubPlan {
     h.part3 = part3.p;
     h.part4 = part4.p;
     h.part5 = part5.p;
+    h.owner = owner.p;
+    h.count = count.p;
     h.n_items = n_items;
     h.n_chunks = n_chunks;
     return h;
@@ -229,9 +235,16 @@ void launch_eval(const DevModel& m, const double* X, const DevScalars* sc, EvalO
                  hipStream_t s);
 void launch_isrc_contrib(int k, const double* isrc, const int32_t* is_dst, double* rf, double* rq,
                          hipStream_t s);
-void launch_reduce_jac(int nse, const int32_t* seg, const double* contrib, const int32_t* slot_diag,
-                       const double* slot_b, const DevScalars* sc, double* csr,
-                       const HubChunks& hub, hipStream_t s);
+struct JacobianArgs {
+  int nse = 0;
+  const int32_t* seg = nullptr;
+  const double* contrib = nullptr;
+  const int32_t* slot_diag = nullptr;
+  const double* slot_b = nullptr;
+  const DevScalars* sc = nullptr;
+  double* csr = nullptr;  // null: no Jacobian wanted
+  HubChunks hub;          // long slots
+};
 struct ResidualArgs {
   int n_unk, m, n_total;
   const int32_t* res_seg;
@@ -258,7 +271,8 @@ struct ResidualArgs {
   DevStatus* st;  // may be null
   HubChunks hub;  // node rows with long residual segments
 };
-void launch_residual(const ResidualArgs& a, hipStream_t s);
+// Jacobian slots and residual rows from the models' contributions, one launch
+void launch_stamp(const JacobianArgs& j, const ResidualArgs& a, hipStream_t s);
 
 template <typename T>
 void launch_lu_refactor(DevLU& lu, const double* csr, T* lu_vals, DevStatus* st, hipStream_t s);

@@ -18,6 +18,7 @@
 #include "block_flags.h"
 #include "circuit.h"
 #include "internal.h"
+#include "lane_value.h"
 
 #include <algorithm>
 #include <cmath>
@@ -762,24 +763,6 @@ __device__ __forceinline__ T group_sum(int start, int end, int lane, F term) {
   return acc;
 }
 
-template <typename F>
-__device__ __forceinline__ double block_max(int start, int end, F term, double* red) {
-  const int t = threadIdx.x;
-  if (t < RB) {
-    double m = 0.0;
-    for (int u = start + t; u < end; u += RB) m = fmax(m, term(u));
-    red[t] = m;
-  }
-  __syncthreads();
-  for (int w = RB / 2; w > 0; w >>= 1) {
-    if (t < w) red[t] = fmax(red[t], red[t + w]);
-    __syncthreads();
-  }
-  const double total = red[0];
-  __syncthreads();
-  return total;
-}
-
 // ---- stamping reductions ----------------------------------------------------
 
 __device__ __forceinline__ double finish_slot(double acc, int s, const int32_t* slot_diag,
@@ -788,47 +771,6 @@ __device__ __forceinline__ double finish_slot(double acc, int s, const int32_t* 
   const double b = slot_b[s];
   if (b != 0.0) acc += b;
   return acc;
-}
-
-// Chunk pre-pass for hub segments: chunk c sums [start[c], end[c]) with one
-// workgroup; the reducing kernels then add a segment's chunk partials in order.
-__global__ void __launch_bounds__(256) k_chunk_sum(const int32_t* __restrict__ cs,
-                                                   const int32_t* __restrict__ ce,
-                                                   const double* __restrict__ v, double* part) {
-  __shared__ double red[RB + 1];
-  const int c = blockIdx.x;
-  const double s = block_sum<double>(cs[c], ce[c], [&](int u) { return v[u]; }, red);
-  if (threadIdx.x == 0) part[c] = s;
-}
-
-// residual rows: sums of rf and rq and max |rf| per chunk
-__global__ void __launch_bounds__(256) k_chunk_res(const int32_t* __restrict__ cs,
-                                                   const int32_t* __restrict__ ce,
-                                                   const double* __restrict__ rf,
-                                                   const double* __restrict__ rq,
-                                                   const double* __restrict__ lr,
-                                                   const double* __restrict__ lq, double* pf,
-                                                   double* pq, double* pm, double* pl,
-                                                   double* plq) {
-  __shared__ double red[RB + 1];
-  const int c = blockIdx.x;
-  const double f = block_sum<double>(cs[c], ce[c], [&](int u) { return rf[u]; }, red);
-  const double q = block_sum<double>(cs[c], ce[c], [&](int u) { return rq[u]; }, red);
-  const double m = block_max(cs[c], ce[c], [&](int u) { return fabs(rf[u]); }, red);
-  double l = 0.0, lc = 0.0;
-  if (lr) {  // uniform across the block
-    l = block_sum<double>(cs[c], ce[c], [&](int u) { return lr[u]; }, red);
-    lc = block_sum<double>(cs[c], ce[c], [&](int u) { return lq[u]; }, red);
-  }
-  if (threadIdx.x == 0) {
-    pf[c] = f;
-    pq[c] = q;
-    pm[c] = m;
-    if (lr) {
-      pl[c] = l;
-      plq[c] = lc;
-    }
-  }
 }
 
 // SpMV rows: sums of a[e] * x[ci[e]] per chunk
@@ -841,33 +783,6 @@ __global__ void __launch_bounds__(256) k_chunk_spmv(const int32_t* __restrict__ 
   const int c = blockIdx.x;
   const double s = block_sum<double>(cs[c], ce[c], [&](int e) { return a[e] * x[ci[e]]; }, red);
   if (threadIdx.x == 0) part[c] = s;
-}
-
-// Blocks [0, n_heavy) finish one hub slot each from its chunk partials; the
-// other blocks reduce one slot per lane.
-__global__ void __launch_bounds__(256) k_reduce_jac(int nse, const int32_t* __restrict__ seg,
-                                                    const double* __restrict__ contrib,
-                                                    const int32_t* __restrict__ slot_diag,
-                                                    const double* __restrict__ slot_b,
-                                                    const DevScalars* __restrict__ sc,
-                                                    double* __restrict__ csr, HubChunks hub) {
-  if ((int)blockIdx.x < hub.n_items) {
-    if (threadIdx.x == 0) {
-      const int s = hub.item[blockIdx.x];
-      double tot = 0.0;
-      for (int c = hub.ptr[blockIdx.x]; c < hub.ptr[blockIdx.x + 1]; ++c) tot += hub.part[c];
-      csr[s] = finish_slot(tot, s, slot_diag, slot_b, sc);
-    }
-    return;
-  }
-  const int n_heavy = hub.n_items;
-  const int s = (blockIdx.x - n_heavy) * blockDim.x + threadIdx.x;
-  if (s >= nse) return;
-  const int u0 = seg[s], u1 = seg[s + 1];
-  if (u1 - u0 > kHeavySegment) return;
-  double acc = 0.0;
-  for (int u = u0; u < u1; ++u) acc += contrib[u];
-  csr[s] = finish_slot(acc, s, slot_diag, slot_b, sc);
 }
 
 // Residual of one node row from its reduced sums (mna_builder.py:1012-1076);
@@ -913,23 +828,140 @@ __device__ __forceinline__ bool finish_row(const ResidualArgs& a, int i, double 
   return !(fchk < tol);
 }
 
-__global__ void __launch_bounds__(256) k_residual(ResidualArgs a) {
-  const HubChunks& hub = a.hub;
-  if ((int)blockIdx.x < hub.n_items) {
-    if (threadIdx.x == 0) {
-      const int i = hub.item[blockIdx.x];
-      double f = 0.0, q = 0.0, mx = 0.0, lf = 0.0, lq = 0.0;
-      for (int c = hub.ptr[blockIdx.x]; c < hub.ptr[blockIdx.x + 1]; ++c) {
-        f += hub.part[c];
-        q += hub.part2[c];
-        mx = fmax(mx, hub.part3[c]);
+// Lane partials of a chunk [u0, u1) of one or two lists in one pass (strided,
+// in order, eight loads in flight), and the first list's largest magnitude.
+template <bool TWO>
+__device__ __forceinline__ void chunk_partials(int u0, int u1, const double* __restrict__ a,
+                                               const double* __restrict__ b, double& sa, double& sb,
+                                               double& mx) {
+  sa = sb = mx = 0.0;
+  for (int e0 = u0 + (int)threadIdx.x; e0 < u1; e0 += 8 * RB) {
+    double x[8], y[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (e0 + t * RB < u1) {
+        x[t] = a[e0 + t * RB];
+        if (TWO) y[t] = b[e0 + t * RB];
+      }
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (e0 + t * RB < u1) {
+        sa += x[t];
+        mx = fmax(mx, fabs(x[t]));
+        if (TWO) sb += y[t];
+      }
+  }
+}
+
+// A chunk's sum is stored for its hub by thread 0, past this XCD's cache (agent
+// scope: the workgroup that reads it may run on another).
+__device__ __forceinline__ void put_partial(double* part, int c, double v) {
+  __hip_atomic_store(&part[c], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// True for the whole workgroup that stored the last of hub h's n chunks; it
+// leaves the counter at zero for the next launch.
+__device__ __forceinline__ bool last_chunk(const HubChunks& hub, int h, int n) {
+  __shared__ int s_last;
+  if (threadIdx.x == 0) {
+    const unsigned int old =
+        __hip_atomic_fetch_add(&hub.count[h], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = old == (unsigned int)(n - 1);
+    if (s_last) __hip_atomic_store(&hub.count[h], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return s_last != 0;
+}
+// Partials [c0, c1) in chunk order (or their maximum) by the first wavefront.
+template <bool MAX>
+__device__ __forceinline__ double partials(const double* part, int c0, int c1) {
+  const int lane = (int)threadIdx.x;
+  double t = 0.0;
+  for (int b = c0; b < c1; b += 64) {
+    double v = 0.0;
+    if (b + lane < c1)
+      v = __hip_atomic_load(&part[b + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int n = c1 - b < 64 ? c1 - b : 64;
+    for (int i = 0; i < n; ++i) {
+      const double x = lane_value(v, i);
+      t = MAX ? fmax(t, x) : t + x;
+    }
+  }
+  return t;
+}
+
+// Stamping in one launch: chunks of the Jacobian's hub slots, chunks of the
+// residual's hub rows, then slots and rows, one per lane.  The workgroup that
+// sums a hub's last chunk finishes the hub, so the chunks run beside the other
+// slots and not before them, and the residual beside the Jacobian.  Bound by
+// the dependent loads of the longest chunk and by launches: against four
+// launches one after another a build of 65k gates went from 108 to 92 us, 2000
+// gates' Newton iterations from 15.0 to 12.3 ms for 30 steps, bit for bit.
+__global__ void __launch_bounds__(256) k_stamp(JacobianArgs j, ResidualArgs a, int njc, int nrc,
+                                               int nj) {
+  __shared__ double red[RB + 1];
+  int b = (int)blockIdx.x;
+  const int tid = (int)threadIdx.x;
+  if (b < njc) {
+    const HubChunks& hub = j.hub;
+    double sum, dummy, mx;
+    chunk_partials<false>(hub.cs[b], hub.ce[b], j.contrib, nullptr, sum, dummy, mx);
+    sum = block_tree<double>(sum, red);
+    const int h = hub.owner[b], c0 = hub.ptr[h], c1 = hub.ptr[h + 1];
+    if (c1 - c0 > 1) {
+      if (tid == 0) put_partial(hub.part, b, sum);
+      if (!last_chunk(hub, h, c1 - c0) || tid >= 64) return;
+      sum = partials<false>(hub.part, c0, c1);
+    }
+    if (tid == 0) {
+      const int s = hub.item[h];
+      j.csr[s] = finish_slot(0.0 + sum, s, j.slot_diag, j.slot_b, j.sc);
+    }
+    return;
+  }
+  b -= njc;
+  if (b < nrc) {
+    const HubChunks& hub = a.hub;
+    const int u0 = hub.cs[b], u1 = hub.ce[b];
+    double f, q, mx, lf = 0.0, lq = 0.0, dummy;
+    chunk_partials<true>(u0, u1, a.rf, a.rq, f, q, mx);
+    f = block_tree<double>(f, red);
+    q = block_tree<double>(q, red);
+    red[tid] = mx;
+    __syncthreads();
+    for (int w = RB / 2; w > 0; w >>= 1) {
+      if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
+      __syncthreads();
+    }
+    mx = red[0];
+    __syncthreads();
+    if (a.lr) {  // uniform across the block
+      chunk_partials<true>(u0, u1, a.lr, a.lq, lf, lq, dummy);
+      lf = block_tree<double>(lf, red);
+      lq = block_tree<double>(lq, red);
+    }
+    const int h = hub.owner[b], c0 = hub.ptr[h], c1 = hub.ptr[h + 1];
+    if (c1 - c0 > 1) {
+      if (tid == 0) {
+        put_partial(hub.part, b, f);
+        put_partial(hub.part2, b, q);
+        put_partial(hub.part3, b, mx);
         if (a.lr) {
-          lf += hub.part4[c];
-          lq += hub.part5[c];
+          put_partial(hub.part4, b, lf);
+          put_partial(hub.part5, b, lq);
         }
       }
+      if (!last_chunk(hub, h, c1 - c0) || tid >= 64) return;
+      f = partials<false>(hub.part, c0, c1);
+      q = partials<false>(hub.part2, c0, c1);
+      mx = partials<true>(hub.part3, c0, c1);
+      if (a.lr) {
+        lf = partials<false>(hub.part4, c0, c1);
+        lq = partials<false>(hub.part5, c0, c1);
+      }
+    }
+    if (tid == 0) {
       double fchk;
-      const bool fail = finish_row(a, i, f, q, mx, lf, lq, fchk);
+      const bool fail = finish_row(a, hub.item[h], 0.0 + f, 0.0 + q, mx, 0.0 + lf, 0.0 + lq, fchk);
       if (a.st) {
         if (fchk > 0.0) atomicMax(&a.st->maxf_bits, dbits(fchk));
         if (fail) atomicAdd(&a.st->res_fail, 1u);
@@ -937,7 +969,19 @@ __global__ void __launch_bounds__(256) k_residual(ResidualArgs a) {
     }
     return;
   }
-  const int i = (blockIdx.x - hub.n_items) * blockDim.x + threadIdx.x;
+  b -= nrc;
+  if (b < nj) {
+    const int s = b * 256 + tid;
+    if (s >= j.nse) return;
+    const int u0 = j.seg[s], u1 = j.seg[s + 1];
+    if (u1 - u0 > kHeavySegment) return;
+    double acc = 0.0;
+    for (int u = u0; u < u1; ++u) acc += j.contrib[u];
+    j.csr[s] = finish_slot(acc, s, j.slot_diag, j.slot_b, j.sc);
+    return;
+  }
+  b -= nj;
+  const int i = b * 256 + tid;
   bool fail = false;
   double fchk = 0.0;
   if (i < a.n_unk) {
@@ -2022,26 +2066,12 @@ void launch_isrc_contrib(int k, const double* isrc, const int32_t* is_dst, doubl
   k_isrc<<<nblk(k, 64), 64, 0, s>>>(k, isrc, is_dst, rf, rq);
 }
 
-void launch_reduce_jac(int nse, const int32_t* seg, const double* contrib, const int32_t* slot_diag,
-                       const double* slot_b, const DevScalars* sc, double* csr,
-                       const HubChunks& hub, hipStream_t s) {
-  if (nse == 0) return;
+void launch_stamp(const JacobianArgs& j, const ResidualArgs& a, hipStream_t s) {
+  const int njc = j.csr ? j.hub.n_chunks : 0, nj = j.csr ? nblk(j.nse, 256) : 0;
+  const int nrc = a.hub.n_chunks, nr = nblk(a.n_unk + a.m, 256);
+  if (njc + nrc + nj + nr == 0) return;
   ktimer_begin(s);
-  if (hub.n_chunks > 0) k_chunk_sum<<<hub.n_chunks, 256, 0, s>>>(hub.cs, hub.ce, contrib, hub.part);
-  k_reduce_jac<<<hub.n_items + nblk(nse, 256), 256, 0, s>>>(nse, seg, contrib, slot_diag, slot_b,
-                                                            sc, csr, hub);
-  ktimer_end(KC_STAMP, s);
-}
-
-void launch_residual(const ResidualArgs& a, hipStream_t s) {
-  const int n = a.n_unk + a.m;
-  if (n == 0) return;
-  const HubChunks& h = a.hub;
-  ktimer_begin(s);
-  if (h.n_chunks > 0)
-    k_chunk_res<<<h.n_chunks, 256, 0, s>>>(h.cs, h.ce, a.rf, a.rq, a.lr, a.lq, h.part, h.part2,
-                                           h.part3, h.part4, h.part5);
-  k_residual<<<h.n_items + nblk(n, 256), 256, 0, s>>>(a);
+  k_stamp<<<njc + nrc + nj + nr, 256, 0, s>>>(j, a, njc, nrc, nj);
   ktimer_end(KC_STAMP, s);
 }
 

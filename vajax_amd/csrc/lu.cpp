@@ -92,12 +92,13 @@ int pattern_upload_csr(vjx_pattern* pat) {
 }
 
 hipError_t HubPlan::build(const int32_t* seg, int n, int nparts) {
-  std::vector<int32_t> hi, hp(1, 0), hcs, hce;
+  std::vector<int32_t> hi, hp(1, 0), hcs, hce, own;
   for (int i = 0; i < n; ++i) {
     const int u0 = seg[i], u1 = seg[i + 1];
     if (u1 - u0 <= kHeavySegment) continue;
     hi.push_back(i);
     for (int c = u0; c < u1; c += kHubChunk) {
+      own.push_back((int32_t)hi.size() - 1);
       hcs.push_back(c);
       hce.push_back(u1 - c > kHubChunk ? c + kHubChunk : u1);
     }
@@ -109,6 +110,9 @@ hipError_t HubPlan::build(const int32_t* seg, int n, int nparts) {
   if (e == hipSuccess) e = ptr.upload(hp);
   if (e == hipSuccess) e = cs.upload(hcs);
   if (e == hipSuccess) e = ce.upload(hce);
+  if (e == hipSuccess) e = owner.upload(own);
+  if (e == hipSuccess) e = count.alloc(n_items);
+  if (e == hipSuccess && n_items) e = hipMemset(count.p, 0, n_items * sizeof(unsigned int));
   if (e == hipSuccess) e = part.alloc(n_chunks);
   if (e == hipSuccess && nparts > 1) e = part2.alloc(n_chunks);
   if (e == hipSuccess && nparts > 2) e = part3.alloc(n_chunks);
