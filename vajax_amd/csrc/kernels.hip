@@ -895,7 +895,7 @@ __device__ __forceinline__ double partials(const double* part, int c0, int c1) {
 // slots and not before them, and the residual beside the Jacobian.  Bound by
 // the dependent loads of the longest chunk and by launches: against four
 // launches one after another a build of 65k gates went from 108 to 92 us, 2000
-// gates' Newton iterations from 15.0 to 12.3 ms for 30 steps, bit for bit.
+// gates' 20 transient steps from 15.0 to 12.3 ms, bit for bit.
 __global__ void __launch_bounds__(256) k_stamp(JacobianArgs j, ResidualArgs a, int njc, int nrc,
                                                int nj) {
   __shared__ double red[RB + 1];

@@ -125,8 +125,7 @@ struct Driver {
     if (!lte_hook) return;
     // the iteration's first kernel cleared st_lte
     launch_lte(n_total, w.Xw.p, w.Vp.p, w.Vmax.p, lte_scale, cfg->reltol, cfg->abstol,
-               w.st_lte.p, s);
-    launch_status_export(w.st_lte.p, nullptr, w.d_hst + 2, s);
+               w.st_lte.p, w.d_hst + 2, s);
   }
 
   hipGraph_t graph = nullptr;
@@ -232,10 +231,8 @@ struct Driver {
       VJX_TRY_HIP(hipEventRecord(ev[3], s));
       ev_pending = true;
     }
-    launch_delta(n_unk, m, n_total, w.delta.p, w.Xw.p, c->d_sc.p, w.st.p, s);
-    launch_update(n_unk, m, n_total, w.delta.p, w.Xw.p, c->d_sc.p, w.st.p, s);
-    launch_noi_clamp(c->n_noi, c->noi_rows.p, w.Xw.p, s);
-    launch_status_export(w.st.p, pat->d_status.p, w.d_hst, s);
+    launch_finish(n_unk, m, n_total, w.delta.p, w.Xw.p, c->d_sc.p, w.st.p, pat->d_status.p,
+                  w.d_hst, c->n_noi, c->noi_rows.p, s);
     return VJX_OK;
   }
 

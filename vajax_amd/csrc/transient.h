@@ -5,10 +5,11 @@
 
 namespace vjx {
 
-void launch_delta(int n_unk, int m, int n_total, const double* delta, const double* X,
-                  const DevScalars* sc, DevStatus* st, hipStream_t s);
-void launch_update(int n_unk, int m, int n_total, const double* delta, double* X,
-                   const DevScalars* sc, const DevStatus* st, hipStream_t s);
+// The end of a Newton iteration: delta test, damped update, noise rows back to
+// their values, and both status records to out (mapped pinned host memory)
+void launch_finish(int n_unk, int m, int n_total, const double* delta, double* X,
+                   const DevScalars* sc, DevStatus* st, const DevStatus* lu_st, DevStatus* out,
+                   int n_noi, const int32_t* noi_rows, hipStream_t s);
 // predictor over the n_total + m unknowns; with floor given, also
 // floor[i] = max(hmrc[i] * reltol, abstol) for i < n_unk
 void launch_predict(int n_total, int m, const double* Xa, const double* h0, const double* h1,
@@ -31,8 +32,9 @@ void launch_gather(int n, const int32_t* idx, const double* a, double* b, hipStr
 void launch_dqdt(int n, double c0, double c1, double d1, double c2, const double* Q,
                  const double* Qp, const double* dQ, const double* Q2, double* out,
                  hipStream_t s);
+// st's record goes to out (mapped pinned host memory) as well
 void launch_lte(int n, const double* Vn, const double* Vp, const double* Vmax, double scale,
-                double reltol, double abstol, DevStatus* st, hipStream_t s);
+                double reltol, double abstol, DevStatus* st, DevStatus* out, hipStream_t s);
 void launch_accept(int n_total, int n_unk, int m, const double* Xw, double* Xa, double* hist_new,
                    double* Vmax, const double* Qn, const double* dQn, double* Qp, double* dQ,
                    double* Q2, const double* mrc, double* hmrc, hipStream_t s);

@@ -23,33 +23,39 @@ __device__ __forceinline__ double jmin(double a, double b) {
   return a < b ? a : b;
 }
 
+constexpr int kStatusLanes = 1024;  // of the kernels that reduce into a status record
+
+__device__ __forceinline__ unsigned long long max_bits(unsigned long long a,
+                                                       unsigned long long b) {
+  return b > a ? b : a;
+}
+
 // delta test of solver_factories.py:283-299
-__global__ void __launch_bounds__(256) k_delta(int n_unk, int m, int n_total,
-                                               const double* __restrict__ delta,
-                                               const double* __restrict__ X,
-                                               const DevScalars* __restrict__ sc, DevStatus* st) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  bool fail = false;
-  double adv = 0.0, ad = 0.0;
-  if (i < n_unk + m) {
+__global__ void __launch_bounds__(1024) k_delta(int n_unk, int m, int n_total,
+                                                const double* __restrict__ delta,
+                                                const double* __restrict__ X,
+                                                const DevScalars* __restrict__ sc, DevStatus* st) {
+  unsigned long long adv = 0, ad = 0;
+  unsigned int fail = 0;
+  for (int i = (int)(blockIdx.x * kStatusLanes + threadIdx.x); i < n_unk + m;
+       i += (int)gridDim.x * kStatusLanes) {
     const double d = delta[i];
     double cd, xr, atol;
     if (i < n_unk) {
       cd = d * sc->nr_damping;
       xr = X[1 + i];
       atol = sc->vntol;
-      adv = fabs(d);
+      adv = max_bits(adv, dbits(fabs(d)));
     } else {
       cd = d;
       xr = X[n_total + (i - n_unk)];
       atol = sc->abstol;
     }
     const double tol = jmax(fabs(xr) * sc->reltol, atol);
-    fail = !(fabs(cd) < tol);
-    ad = fabs(d);
+    fail += !(fabs(cd) < tol);
+    ad = max_bits(ad, dbits(fabs(d)));
   }
-  block_flags(dbits(adv), dbits(ad), fail ? 1u : 0u, &st->maxdv_bits, &st->maxdelta_bits,
-              &st->delta_fail);
+  block_flags(adv, ad, fail, &st->maxdv_bits, &st->maxdelta_bits, &st->delta_fail);
 }
 
 // damped update of solver_factories.py:301-309
@@ -66,6 +72,81 @@ __global__ void __launch_bounds__(256) k_update(int n_unk, int m, int n_total,
   } else {
     const int j = n_total + (i - n_unk);
     X[j] = X[j] + delta[i];
+  }
+}
+
+// k_delta, k_update and k_status_export in one workgroup, for systems of up to
+// kFinishMax unknowns: the maxima go through LDS instead of memory, the deltas
+// and the iterate stay in registers between test and update, and the same
+// thread that has the counts exports the records.
+constexpr int kFinishEach = 8;
+constexpr int kFinishMax = kStatusLanes * kFinishEach;
+__global__ void __launch_bounds__(1024) k_finish(int n_unk, int m, int n_total,
+                                                 const double* __restrict__ delta, double* X,
+                                                 const DevScalars* __restrict__ sc, DevStatus* st,
+                                                 const DevStatus* __restrict__ lu_st,
+                                                 DevStatus* out) {
+  __shared__ unsigned long long s_adv, s_ad;
+  __shared__ unsigned int s_fail;
+  const int tid = (int)threadIdx.x;
+  if (tid == 0) {
+    s_adv = s_ad = 0;
+    s_fail = 0;
+  }
+  const int n = n_unk + m;
+  double d[kFinishEach], x[kFinishEach];
+#pragma unroll
+  for (int u = 0; u < kFinishEach; ++u) {
+    const int i = tid + u * kStatusLanes;
+    if (i < n) {
+      d[u] = delta[i];
+      x[u] = X[i < n_unk ? 1 + i : n_total + (i - n_unk)];
+    }
+  }
+  unsigned long long adv = 0, ad = 0;
+  unsigned int fail = 0;
+#pragma unroll
+  for (int u = 0; u < kFinishEach; ++u) {
+    const int i = tid + u * kStatusLanes;
+    if (i < n) {
+      const bool node = i < n_unk;
+      const double cd = node ? d[u] * sc->nr_damping : d[u];
+      const double tol = jmax(fabs(x[u]) * sc->reltol, node ? sc->vntol : sc->abstol);
+      fail += !(fabs(cd) < tol);
+      ad = max_bits(ad, dbits(fabs(d[u])));
+      if (node) adv = max_bits(adv, dbits(fabs(d[u])));
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    adv = max_bits(adv, __shfl_xor(adv, o));
+    ad = max_bits(ad, __shfl_xor(ad, o));
+    fail += __shfl_xor(fail, o);
+  }
+  __syncthreads();
+  if ((tid & 63) == 0) {
+    atomicMax(&s_adv, adv);
+    atomicMax(&s_ad, ad);
+    atomicAdd(&s_fail, fail);
+  }
+  __syncthreads();
+  const double vs = jmin(1.0, sc->max_step / jmax(bitsd(s_adv), 1e-30));
+#pragma unroll
+  for (int u = 0; u < kFinishEach; ++u) {
+    const int i = tid + u * kStatusLanes;
+    if (i < n_unk)
+      X[1 + i] = x[u] + d[u] * vs * sc->nr_damping;
+    else if (i < n)
+      X[n_total + (i - n_unk)] = x[u] + d[u];
+  }
+  if (tid == 0) {
+    DevStatus r = *st;
+    r.maxdv_bits = s_adv;
+    r.maxdelta_bits = s_ad;
+    r.delta_fail = s_fail;
+    *st = r;
+    out[0] = r;
+    out[1] = *lu_st;
   }
 }
 
@@ -143,21 +224,28 @@ __global__ void k_dqdt(int n, double c0, double c1, double d1, double c2,
 }
 
 // LTE ratio of adaptive.py:254-271
-__global__ void __launch_bounds__(256) k_lte(int n, const double* __restrict__ Vn,
+__global__ void __launch_bounds__(1024) k_lte(int n, const double* __restrict__ Vn,
                                              const double* __restrict__ Vp,
                                              const double* __restrict__ Vmax, double scale,
-                                             double reltol, double abstol, DevStatus* st) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double r = 0.0;
-  if (i < n) {
+                                             double reltol, double abstol, DevStatus* st,
+                                             DevStatus* out) {
+  unsigned long long top = 0;
+  for (int i = (int)(blockIdx.x * kStatusLanes + threadIdx.x); i < n;
+       i += (int)gridDim.x * kStatusLanes) {
     const double lte = (Vn[i] - Vp[i]) * scale;
     const double vc = jmax(fabs(Vn[i]), fabs(Vp[i]));
     const double vs = jmax(Vmax[i], vc);
     const double tol = reltol * vs + abstol;
-    r = fabs(lte) / tol;
+    double r = fabs(lte) / tol;
     if (r != r) r = __longlong_as_double(0x7ff8000000000000LL);
+    top = max_bits(top, dbits(r));
   }
-  block_flags(dbits(r), 0, 0u, &st->maxf_bits, nullptr, nullptr);
+  block_flags(top, 0, 0u, &st->maxf_bits, nullptr, nullptr);
+  if (out && threadIdx.x == 0) {  // the only workgroup
+    DevStatus r = *st;
+    r.maxf_bits = __hip_atomic_load(&st->maxf_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *out = r;
+  }
 }
 
 // state update on use_new_solution (full_mna.py:2078-2113)
@@ -191,15 +279,33 @@ __global__ void k_output(int n_total, int m, const double* __restrict__ Xa,
 
 inline int nb(long long n, int b = 256) { return (int)((n + b - 1) / b); }
 
+// A status kernel's workgroups each end with one atomic a value on the same
+// cache line, and those run one after another (about 10 ns each), so its
+// workgroups have 1024 lanes and there are at most 128 of them: at 130k
+// unknowns k_delta 6.8 us and k_lte 4.5 us (14.3 and 8.0 with 509 workgroups of 256).
+inline int status_blocks(int n) {
+  const int b = (n + kStatusLanes - 1) / kStatusLanes;
+  return b < 128 ? b : 128;
+}
+
 }  // namespace
 
-void launch_delta(int n_unk, int m, int n_total, const double* delta, const double* X,
-                  const DevScalars* sc, DevStatus* st, hipStream_t s) {
-  k_delta<<<nb(n_unk + m), 256, 0, s>>>(n_unk, m, n_total, delta, X, sc, st);
-}
-void launch_update(int n_unk, int m, int n_total, const double* delta, double* X,
-                   const DevScalars* sc, const DevStatus* st, hipStream_t s) {
-  k_update<<<nb(n_unk + m), 256, 0, s>>>(n_unk, m, n_total, delta, X, sc, st);
+void launch_finish(int n_unk, int m, int n_total, const double* delta, double* X,
+                   const DevScalars* sc, DevStatus* st, const DevStatus* lu_st, DevStatus* out,
+                   int n_noi, const int32_t* noi_rows, hipStream_t s) {
+  const int n = n_unk + m;
+  // One workgroup up to eight unknowns a lane (noise rows are reset between
+  // update and export, so circuits with them keep the launches): the ring of
+  // 101 stages 13.0 -> 12.6 ms, even at 4 300 unknowns (14.0 ms); beyond, one
+  // compute unit's loads would be the bound.
+  if (n <= kFinishMax && n_noi == 0) {
+    k_finish<<<1, kStatusLanes, 0, s>>>(n_unk, m, n_total, delta, X, sc, st, lu_st, out);
+    return;
+  }
+  k_delta<<<status_blocks(n), kStatusLanes, 0, s>>>(n_unk, m, n_total, delta, X, sc, st);
+  k_update<<<nb(n), 256, 0, s>>>(n_unk, m, n_total, delta, X, sc, st);
+  launch_noi_clamp(n_noi, noi_rows, X, s);
+  launch_status_export(st, lu_st, out, s);
 }
 void launch_predict(int n_total, int m, const double* Xa, const double* h0, const double* h1,
                     const double* h2, double a0, double a1, double a2, int can_predict, double* Vp,
@@ -265,8 +371,14 @@ void launch_dqdt(int n, double c0, double c1, double d1, double c2, const double
   if (n) k_dqdt<<<nb(n), 256, 0, s>>>(n, c0, c1, d1, c2, Q, Qp, dQ, Q2, out);
 }
 void launch_lte(int n, const double* Vn, const double* Vp, const double* Vmax, double scale,
-                double reltol, double abstol, DevStatus* st, hipStream_t s) {
-  k_lte<<<nb(n), 256, 0, s>>>(n, Vn, Vp, Vmax, scale, reltol, abstol, st);
+                double reltol, double abstol, DevStatus* st, DevStatus* out, hipStream_t s) {
+  if (n <= kFinishMax) {
+    k_lte<<<1, kStatusLanes, 0, s>>>(n, Vn, Vp, Vmax, scale, reltol, abstol, st, out);
+  } else {
+    k_lte<<<status_blocks(n), kStatusLanes, 0, s>>>(n, Vn, Vp, Vmax, scale, reltol, abstol, st,
+                                                    nullptr);
+    launch_status_export(st, nullptr, out, s);
+  }
 }
 void launch_accept(int n_total, int n_unk, int m, const double* Xw, double* Xa, double* hist_new,
                    double* Vmax, const double* Qn, const double* dQn, double* Qp, double* dQ,
