@@ -115,6 +115,21 @@ def test_front_program_on_the_cpu(name):
     assert _residual(ip, ix, a, lu.solve_cpu(a, b, 1), b) <= 65 * 6e-8 * 4
 
 
+@pytest.mark.parametrize("rows,front", [(64, True), (65, False)])
+def test_later_analyses_of_a_handle_keep_its_kind_of_program(rows, front):
+    ip, ix, a = _csr(_dense(rows, 9))
+    lu = SparseLU(ip, ix)
+    b = np.random.default_rng(3).standard_normal(rows)
+    for width in (None, None, 8):  # a setter between the second and the third
+        if width:
+            lu.set_band_width(width)
+        lu.analyze(a)
+        lu.check_schedules()
+        assert (lu.info()["fact_task_targets"] == 0) == front
+        assert _residual(ip, ix, a, lu.solve_cpu(a, b), b) <= 65 * 2.3e-16 * 4
+        a = a * np.random.default_rng(4).uniform(0.9, 1.1, len(a))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(CASES))
 def test_front_program_matches_its_cpu_execution(name):

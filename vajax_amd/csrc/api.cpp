@@ -107,6 +107,13 @@ int vjx_lu_analyze(vjx_pattern* pat, const double* data_host) {
       fresh = std::move(alt);
     }
   }
+  // A system without a front program is ordered and pivoted twice, once to
+  // find that out; the handle's later analyses (the autotuner's widths, a
+  // re-pivot in the Newton loop) go straight to the band programs until a
+  // setter changes what is analysed.  (Not after a front program: the pivots
+  // of one bad iterate say little about the next.)
+  if (o.fronts && !fresh.front.on() && !(pat->lu.analyzed && pat->lu.sym.front.on()))
+    pat->opts.fronts = false;
   pat->lu.sym = std::move(fresh);
   pat->analyze_seconds =
       std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -242,6 +249,7 @@ int vjx_pattern_set_band_width(vjx_pattern* pat, int32_t width) {
   if (pat->opts.band_width != width) {
     pat->opts.band_width = width;
     // the schedules change: analyse again on next use
+    pat->opts.fronts = true;
     pat->lu.analyzed = false;
     pat->lu.factored_prec = -1;
     pat->uploaded = false;
@@ -260,6 +268,7 @@ int vjx_pattern_set_ordering(vjx_pattern* pat, int32_t ordering, int32_t nd_leaf
   if (pat->opts.ordering != ordering || (nd && pat->opts.nd_leaf != nd_leaf)) {
     pat->opts.ordering = ordering;
     if (nd) pat->opts.nd_leaf = nd_leaf;
+    pat->opts.fronts = true;
     pat->lu.analyzed = false;
     pat->lu.factored_prec = -1;
     pat->uploaded = false;
@@ -284,6 +293,7 @@ int vjx_pattern_set_dense(vjx_pattern* pat, int32_t min_rows, double density) {
   if (pat->opts.dense_min != min_rows || pat->opts.dense_density != density) {
     pat->opts.dense_min = min_rows;
     pat->opts.dense_density = density;
+    pat->opts.fronts = true;
     pat->lu.analyzed = false;
     pat->lu.factored_prec = -1;
     pat->uploaded = false;

@@ -226,7 +226,8 @@ struct AnalyzeOptions {
   double dense_density = 0.4;
   int solve_band_width = 0;   // solve bands (0: band_width)
   // front program where the matrix has one and band_width > 0 (else, and for
-  // the natural order, the band or level programs)
+  // the natural order, the band or level programs); a handle clears it when an
+  // analysis found none
   bool fronts = true;
   int max_band_tasks = 2048;  // workgroups per band launch
   // abandon the analysis once L + U hold more entries than this (0: no
