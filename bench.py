@@ -148,6 +148,13 @@ def kernel_bytes(topo, info, precision: str):
     # operands it gathers are counted once per row), per row the item, row
     # pointers, the right-hand side / result and the pivot
     solves = (4 + vb) * offd + (4 + 8 + 3 * vb) * 2 * n
+    if front_program(info):
+        # dense fronts: A's entries (value, index, place) read and the LU
+        # entries written once; a solve reads them once, without indices.  The
+        # update blocks that fronts hand to their parents are not counted.
+        lu_tasks = (8 + 4 + 2) * nse + vb * nnz_lu
+        lu_gather = lu_schur = 0
+        solves = vb * offd + (8 + 3 * vb) * 2 * n
     if precision == "f32":       # second solve of the refinement step + FP64 SpMV
         solves = 2 * solves
     # dense trailing block: its slots gathered and written back, the
@@ -160,7 +167,16 @@ def kernel_bytes(topo, info, precision: str):
             "lu_dense": lu_dense}
 
 
-KERNEL_NAMES = {"eval": "k_eval<MOSFET> (+R/C)", "stamp": "k_chunk_sum/k_reduce_jac/k_chunk_res/k_residual",
+def front_program(info):
+    """Whether the LU runs as dense fronts (no scalar targets in its program)."""
+    return info["fact_task_targets"] == 0 and info["n_updates"] > 0
+
+
+FRONT_NAMES = {"lu_gather": "k_front_prep (source rows)",
+               "lu_tasks": "k_front_small/k_front_large/k_front_tiny",
+               "solve_tasks": "k_front_fwd/k_front_bwd/k_front_tiny",
+               "solve_hub": "k_front_single (source columns)"}
+KERNEL_NAMES = {"eval": "k_eval<MOSFET> (+R/C)", "stamp": "k_stamp",
                 "lu_gather": "k_lu_gather", "lu_tasks": "k_lu_band_lds (band tasks)",
                 "lu_schur": "k_lu_wide (Schur step)",
                 "lu_scale": "k_lu_scale (level programs only)", "solve_tasks": "k_tri_band_lde (forward + backward)",
@@ -170,14 +186,16 @@ KERNEL_NAMES = {"eval": "k_eval<MOSFET> (+R/C)", "stamp": "k_chunk_sum/k_reduce_
 
 # kernel class -> kernel-name prefixes in the rocprofv3 traffic summaries
 TRAFFIC_KERNELS = {
-    "eval": ["k_eval<"], "stamp": ["k_reduce_jac", "k_residual", "k_chunk_sum", "k_chunk_res"],
-    "lu_gather": ["k_lu_gather<double>"], "lu_tasks": ["k_lu_band_lds<double", "k_lu_band<double>"],
+    "eval": ["k_eval<"], "stamp": ["k_stamp"],
+    "lu_gather": ["k_lu_gather<double>", "k_front_prep<double>"],
+    "lu_tasks": ["k_lu_band_lds<double", "k_lu_band<double>", "k_front_small<double",
+                 "k_front_large<double"],
     "lu_schur": ["k_lu_wide<double"], "lu_scale": ["k_lu_scale<double>"],
-    "solve_tasks": ["k_tri_band_lde<double", "k_tri_band<double"],
+    "solve_tasks": ["k_tri_band_lde<double", "k_tri_band<double", "k_front_bwd<double>"],
     "lu_dense": ["k_dgemm_sub", "k_dense_panel", "k_dense_diag"]}
 
 
-def measured_traffic(args, cls):
+def measured_traffic(args, cls, front):
     """HBM bytes per dispatch of a kernel class (dispatch-weighted mean over
     its kernels) from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary
     of this workload, scaled by the copy-kernel calibration; None when no
@@ -187,7 +205,10 @@ def measured_traffic(args, cls):
         return None
     with open(path) as fh:
         data = json.load(fh)["kernels"]
-    ks = [v for k, v in data.items() if any(k.startswith(p) for p in TRAFFIC_KERNELS.get(cls, []))]
+    prefixes = TRAFFIC_KERNELS.get(cls, [])
+    if cls.startswith("lu_") or cls.startswith("solve_"):  # the program that ran
+        prefixes = [p for p in prefixes if p.startswith("k_front") == front]
+    ks = [v for k, v in data.items() if any(k.startswith(p) for p in prefixes)]
     n = sum(k["dispatches"] for k in ks)
     if n == 0:
         return None
@@ -782,12 +803,13 @@ def main():
     per_iter = ({"build": ph["build_ms"] / iters, "lu": ph["lu_ms"] / iters,
                  "solve": ph["solve_ms"] / iters} if ph else {})
     kb = kernel_bytes(topo, lu_info, args.precision)
+    names = {**KERNEL_NAMES, **(FRONT_NAMES if front_program(lu_info) else {})}
     for name, kt in (ph["kernels"].items() if ph else ()):
         if kt["launches"] == 0:
             continue
         avg_ms = kt["ms"] / kt["launches"]
         per_launch = kb[name] / (kt["launches"] / iters)
-        kernels[name] = {"kernel": KERNEL_NAMES[name], "ms_per_newton_iter": round(kt["ms"] / iters, 4),
+        kernels[name] = {"kernel": names[name], "ms_per_newton_iter": round(kt["ms"] / iters, 4),
                          "launches_per_newton_iter": round(kt["launches"] / iters, 2),
                          "avg_launch_us": round(avg_ms * 1e3, 2),
                          "alg_bytes_per_launch": int(per_launch),
@@ -796,7 +818,7 @@ def main():
     if kernels:
         dom = max(kernels, key=lambda k: kernels[k]["ms_per_newton_iter"])
         d = kernels[dom]
-        traffic = measured_traffic(args, dom)
+        traffic = measured_traffic(args, dom, front_program(lu_info))
         roofline = {
             "bound": "hbm",
             "kernel": d["kernel"],

@@ -128,11 +128,13 @@ typedef struct {
    * distinct block patterns, each analysed once and shared */
   int32_t n_blocks;
   int32_t n_block_patterns;
-  /* triangular-solve band programs: bands (launches) and hub rows */
+  /* triangular-solve band programs: bands (launches) and hub rows; a front
+   * program (dense fronts of up to 64 rows on the elimination tree, taken
+   * whenever every front fits) counts its stages here and in *_launches */
   int32_t fwd_bands, bwd_bands, fwd_hub_rows, bwd_hub_rows;
   /* refactorisation band program: update contributions and targets run by
    * the band tasks and by the Schur steps (all in the tasks' counts when the
-   * level program is used) */
+   * level program is used; no targets when a front program is) */
   int64_t fact_task_updates, fact_schur_updates, fact_task_targets, fact_schur_targets;
   /* analysis time in ms: ordering, pivoting, LU pattern, refactorisation
    * program, solve programs (single-block systems; zero for packed batches) */
@@ -190,8 +192,9 @@ int vjx_pattern_set_fill_limit(vjx_pattern* pat, int64_t max_lu_nnz);
  * cores; min_rows 0 = never (default 96, 0.4).  A change drops the analysis.
  * No counterpart in the reference (a supernode-shape choice). */
 int vjx_pattern_set_dense(vjx_pattern* pat, int32_t min_rows, double density);
-/* Autotuner of the launch plan: with the matrix data_dev (device), time the
- * numeric refactorisation for refactorisation bands of 12, 16 and 24 pivot
+/* Autotuner of the launch plan.  A front program has one plan: its
+ * refactorisation and solve are timed once.  Otherwise, with the matrix
+ * data_dev (device), time the numeric refactorisation for refactorisation bands of 12, 16 and 24 pivot
  * levels (a fresh analysis each: same ordering and pivots) and each LU
  * band-task pipeline, keep the fastest, then time the triangular solves for
  * band widths 8..64 and keep the fastest (solve results do not depend on

@@ -202,13 +202,13 @@ struct HubPlan {
 // ----- per-kernel timing (profiling passes only, never under graph capture) --
 enum KernelClass {
   KC_EVAL = 0,     // k_eval<model>
-  KC_STAMP,        // chunk pre-passes + k_reduce_jac + k_residual
-  KC_LU_GATHER,    // k_lu_gather
-  KC_LU_TASKS,     // k_lu_band (and level launches of the level program)
+  KC_STAMP,        // k_stamp
+  KC_LU_GATHER,    // k_lu_gather, k_front_prep
+  KC_LU_TASKS,     // k_front_*, k_lu_band (and level launches of the level program)
   KC_LU_SCHUR,     // k_lu_wide of a band's Schur step
   KC_LU_SCALE,     // k_lu_scale
-  KC_TRI_TASKS,    // k_tri_band (and level launches of the level program)
-  KC_TRI_HUB,      // chunked hub rows of the solves
+  KC_TRI_TASKS,    // k_front_fwd / k_front_bwd, k_tri_band (and level launches of the level program)
+  KC_TRI_HUB,      // chunked hub rows of the solves, k_front_single
   KC_LU_DENSE,     // dense trailing block: gathers, MFMA products, panels, write-back
   KC_COUNT
 };

@@ -13,7 +13,10 @@
 // behind.  Nothing in it has to start at zero: the forward solve writes every
 // intermediate entry before it is read, and every hub partial is written
 // before its row is finished.  Calls that overlap on one GPU (two host threads,
-// or two streams) race on the array.
+// or two streams) race on the array.  Of a front program's solve the fronts'
+// contributions and the source columns' chunk sums stay in the handle's own
+// buffers, which its analysis allocated, so a call that overlaps another solve
+// of the same handle races on those as well.
 #include <mutex>
 
 #include "circuit.h"
